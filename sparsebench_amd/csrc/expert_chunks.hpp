@@ -393,6 +393,49 @@ __host__ __device__ __forceinline__ bool balanced_chunk_tile(int bid, int chunks
   return true;
 }
 
+// Narrow tiles: row-block tiles of 64, 128 or 256 columns for layouts with
+// so few live row blocks that the wide tiles leave CUs idle (decode steps: a
+// few rows in each of a few experts). Such a tile is bound by its CU's stream
+// of weights: one CU takes in at most about 53 GB/s of L2 misses (a 128-byte
+// line every 5 cycles, with 32 KB in flight or 128; 128 GB/s when L2 holds
+// the data), so the stage takes as long as one tile's weights at that rate
+// until about 128 CUs stream. The width is the smallest at which every tile
+// has a CU of its own; past that tiles queue, and their shorter row segments
+// cost HBM efficiency when all CUs stream (D = 1024, F = 4096, E = 64, 320
+// tiles of 128: DSD 66 us against 53 for the 512-wide tiles' halves). The
+// DSD's 256-wide tiles are left to the row blocks' halves and the expert
+// tiles, which are as wide (84 against 94 us with 64 row blocks).
+// Against the wide tiles alone (stage times, graph replay):
+//   D = 1024, F = 4096, E = 64:  T = 1 SDD 18.2 -> 8.9, DSD 41.3 -> 19.5 us;
+//     T = 8 26.3 -> 23.9, 44.8 -> 26.0; T = 32 Zipf DSD 49.5 -> 39.3
+//   D = 4096, F = 14336, E = 8:  T = 1 72.4 -> 43.1, 192.7 -> 66;
+//     T = 32 DSD 184 -> 142
+//   D = 2048, F = 768, E = 128:  T = 8 21.5 -> 13.6, 15.0 -> 13.6
+constexpr int kSddWidestNarrow = 256, kDsdWidestNarrow = 128;
+
+// The narrow tiles' width, or 0 for the wide tiles.
+__host__ __device__ __forceinline__ int narrow_width(int live_rb, int columns, int widest, int cus) {
+  if (live_rb <= 0 || live_rb > cus) return 0;
+#pragma unroll
+  for (int log_bn = 6; log_bn <= 8; ++log_bn)  // shifts: a division is a long sequence at every tile's start
+    if ((1 << log_bn) <= widest && static_cast<int64_t>(live_rb) * (columns >> log_bn) <= cus) return 1 << log_bn;
+  return 0;
+}
+
+// Workgroup bid's narrow tile (rb >= live_rb: none), slice by slice within a
+// row block. Workgroups go to the XCDs round-robin, so with 16, 24, ...
+// slices an expert's row blocks meet a slice's weights in one XCD's L2 and
+// each XCD streams a part of every expert (D = 4096, F = 14336, E = 8,
+// T = 32: DSD 141.5 us, against 150 with an expert an XCD); for other counts
+// each XCD gets a contiguous range of tiles (D = 1024, F = 1536, E = 32,
+// T = 1024: DSD 23.0 us against 27.3 with one of 8 slices an XCD; with 6
+// slices an expert's row blocks would not meet at all).
+__host__ __device__ __forceinline__ void narrow_tile_for(int bid, int live_rb, int slices, int* rb, int* slice) {
+  const int tile = slices % kNumXcd == 0 && slices > kNumXcd ? bid : xcd_remap(bid, live_rb * slices);
+  *rb = uniform(tile / slices);
+  *slice = uniform(tile - tile / slices * slices);
+}
+
 // Which tiling computes a stage of the MoE layer: expert chunks or row
 // blocks. Every workgroup of the stage's kernel makes the same choice from
 // the same counts, so it costs no host sync.

@@ -44,6 +44,7 @@
 // vmcnt(0) after every step's barrier from the compiler (its LDS-DMA alias
 // tracking loses the stages apart), which serialises its loads and MFMAs.
 
+#include "chunk_tiles.hpp"
 #include "expert_chunks.hpp"
 #include "gelu.hpp"
 #include "gemm_dma.hpp"
@@ -79,12 +80,6 @@ template <int R, int BN, int WAVES, int STAGES>
 using DsdCfg = DmaCfg<32 * R, BN, 32, STAGES, (WAVES == 8 && R % 2 == 0) ? 2 : 1,
                       (WAVES == 8 && R % 2 == 0) ? WAVES / 2 : WAVES, 0, 2, 5, 1, STAGES == 4 ? 1 : 0>;
 
-// A tile configuration cut to R row groups (R a multiple of its rows of
-// waves, WM: DmaCfg asserts that each wave owns whole 32-row groups).
-template <class Cfg, int R>
-using RowsCfg = DmaCfg<32 * R, Cfg::BN, Cfg::BK, Cfg::STAGES, Cfg::WM, Cfg::WN, Cfg::CPA, Cfg::CPB, Cfg::PIPE,
-                       Cfg::EPI_PARTS, Cfg::APAIR ? 1 : 0, Cfg::BSTAGES == Cfg::STAGES ? 0 : Cfg::BSTAGES>;
-
 // LDS of the expert tiles of a kernel: the largest over its tile heights.
 template <int BN, int WAVES, int STAGES, int R>
 constexpr int chunk_lds_bytes() {
@@ -99,85 +94,71 @@ constexpr int chunk_lds_bytes() {
 
 constexpr int max_int(int a, int b) { return a > b ? a : b; }
 
-// f(integral_constant<int, R>) for the chunk's R in 1 .. RMAX.
-template <int RMAX, class F>
-__device__ __forceinline__ void with_groups(int groups, F&& f) {
-  static_for<1, RMAX + 1>([&](auto rc) {
+// --------------------------------------------------------- narrow tiles ---
+
+// K steps of 64 through as deep a ring as 160 KB hold (up to 8 stages). The
+// computing waves are laid out to read each fragment as few times as can be;
+// the workgroup's other waves share the loads.
+template <int R, int BN, int WAVES>
+struct NarrowShape {
+  static constexpr int WN = (BN == 256 && WAVES == 8 && R % 2 == 0) ? 4 : (BN / 32 < WAVES ? BN / 32 : WAVES);
+  static constexpr int kRowWaves = WAVES / WN;
+  static constexpr int WM = (R % 4 == 0 && kRowWaves >= 4) ? 4 : (R % 2 == 0 && kRowWaves >= 2) ? 2 : 1;
+  static constexpr int XW = WAVES - WM * WN;
+  static constexpr int kStage = (R * 4096 + 1024 * WAVES - 1) / (1024 * WAVES) * (1024 * WAVES) + BN * 128;
+  static constexpr int kFit = 160 * 1024 / kStage;
+  using Cfg = std::conditional_t<(R == 4 && BN == 256 && WAVES == 8), SddHalfTile,
+                                 DmaCfg<32 * R, BN, 64, (kFit < 8 ? kFit : 8), WM, WN, 0, 2, 5, 1, 0, 0, XW>>;
+  static_assert(Cfg::kThreads == 64 * WAVES, "the kernel's workgroup");
+};
+
+template <int WAVES, int WIDEST, int R = 4>
+constexpr int narrow_lds_bytes() {
+  constexpr int own = max_int(max_int(NarrowShape<R, 64, WAVES>::Cfg::kLdsAlloc, NarrowShape<R, 128, WAVES>::Cfg::kLdsAlloc),
+                              NarrowShape<R, WIDEST, WAVES>::Cfg::kLdsAlloc);
+  if constexpr (R == 1) return own;
+  else return max_int(own, narrow_lds_bytes<WAVES, WIDEST, R - 1>());
+}
+
+// f(Tag<configuration>) for a narrow tile of `groups` row groups and `bn` columns.
+template <int WAVES, int WIDEST, class F>
+__device__ __forceinline__ void with_narrow(int groups, int bn, F&& f) {
+  with_groups<4>(groups, [&](auto rc) {
     constexpr int R = decltype(rc)::value;
-    if (groups == R) f(rc);
+    if (bn == 64) f(Tag<typename NarrowShape<R, 64, WAVES>::Cfg>{});
+    else if (bn == 128) f(Tag<typename NarrowShape<R, 128, WAVES>::Cfg>{});
+    else if constexpr (WIDEST >= 256) f(Tag<typename NarrowShape<R, 256, WAVES>::Cfg>{});
   });
+}
+
+// The row block of workgroup bid's narrow tile. An expert of one row block
+// stops at its last real 32-row group; the row blocks of a larger one are
+// whole, unless the stage's choice is the expert tiles (expert_choice(),
+// asked only then), whose outputs end at an expert's real rows.
+template <class Choice>
+__device__ __forceinline__ bool narrow_chunk(int bid, int live_rb, int slices,
+                                             const int32_t* __restrict__ row_block_expert,
+                                             const int32_t* __restrict__ tokens_per_expert,
+                                             const int32_t* __restrict__ padded_offsets, int32_t num_experts,
+                                             int32_t max_row_blocks, bool cut_single, const Choice& expert_choice,
+                                             Chunk* ch, int* slice) {
+  int rb;
+  narrow_tile_for(bid, live_rb, slices, &rb, slice);
+  if (rb >= live_rb || rb >= max_row_blocks) return false;
+  const int32_t expert = __builtin_amdgcn_readfirstlane(row_block_expert[rb]);
+  if (expert < 0 || expert >= num_experts) return false;
+  const int32_t n = __builtin_amdgcn_readfirstlane(tokens_per_expert[expert]);
+  const int32_t row = rb * kBS - __builtin_amdgcn_readfirstlane(padded_offsets[expert]);  // the block's first row of it
+  if (row < 0 || row >= n) return false;  // not a routing layout
+  const bool cut = n <= kBS ? cut_single : expert_choice();
+  ch->expert = expert;
+  ch->row0 = rb * kBS;
+  ch->rows = cut ? min(n - row, kBS) : kBS;
+  ch->groups = (ch->rows + 31) / 32;
+  return true;
 }
 
 // ------------------------------------------------------------------ SDD ---
-
-template <class Cfg>
-struct SddChunkSrc {
-  __amdgpu_buffer_rsrc_t x_rsrc, w_rsrc;
-  uint32_t a_off[Cfg::kAInstr];
-  uint32_t b_off[Cfg::kBInstr];
-  uint32_t b_step_bytes;
-  __device__ __forceinline__ uint32_t a_voff(int q) const { return a_off[q]; }
-  __device__ __forceinline__ uint32_t b_voff(int q) const { return b_off[q]; }
-  __device__ __forceinline__ void a_src(int t, __amdgpu_buffer_rsrc_t* r, uint32_t* s) const {
-    *r = x_rsrc;
-    *s = static_cast<uint32_t>(t) * (Cfg::BK * 2);
-  }
-  __device__ __forceinline__ void b_src(int t, __amdgpu_buffer_rsrc_t* r, uint32_t* s) const {
-    *r = w_rsrc;
-    *s = static_cast<uint32_t>(t) * b_step_bytes;
-  }
-};
-
-struct SddArgs {
-  const uint16_t* x;
-  const uint16_t* w1;
-  const int32_t* row_token;
-  uint16_t* out;
-  int32_t num_tokens, d_model, ffn_dim;
-  int32_t apply_gelu;
-};
-
-template <class Cfg>
-__device__ __forceinline__ void sdd_chunk_tile(uint8_t* __restrict__ lds, const SddArgs& a, const Chunk& ch, int n0) {
-  using ML = DmaMainloop<Cfg>;
-  SddChunkSrc<Cfg> src;
-  src.x_rsrc = make_rsrc(a.x, static_cast<uint32_t>(a.num_tokens) * static_cast<uint32_t>(a.d_model) * 2u);
-  src.w_rsrc = make_rsrc(a.w1 + static_cast<int64_t>(ch.expert) * a.d_model * a.ffn_dim,
-                         static_cast<uint32_t>(a.d_model) * static_cast<uint32_t>(a.ffn_dim) * 2u);
-  src.b_step_bytes = static_cast<uint32_t>(Cfg::BK) * static_cast<uint32_t>(a.ffn_dim) * 2u;
-  const ADmaPos<Cfg> ap;
-#pragma unroll
-  for (int q = 0; q < Cfg::kAInstr; ++q) {
-    const int j = ap.row[q];  // row of the chunk; rows past BM belong to the rounded-up DMA area
-    const int32_t tok = j < ch.rows ? a.row_token[ch.row0 + j] : -1;
-    src.a_off[q] = (tok >= 0 && tok < a.num_tokens)
-                       ? static_cast<uint32_t>(tok) * static_cast<uint32_t>(a.d_model) * 2u + ap.chunk[q] * 16u
-                       : kOutOfRange;
-  }
-  const BDmaPos<Cfg> bp;
-#pragma unroll
-  for (int q = 0; q < Cfg::kBInstr; ++q)
-    src.b_off[q] = (static_cast<uint32_t>(bp.row[q]) * a.ffn_dim + n0 + bp.col[q]) * 2u;
-
-  typename ML::Acc acc;
-  ML::run(lds, src, a.d_model / Cfg::BK, acc);
-
-  // Padded row p -> row block p / 128, whose blocks are (p / 128) * F/128 + f/128.
-  const int64_t ffn_blocks = a.ffn_dim / kBS;
-  static_for<0, Cfg::EPI_PARTS>([&](auto pc) {
-    constexpr int P = decltype(pc)::value;
-    if (a.apply_gelu)
-      ML::template stage_part<P>(lds, acc, [](float v) { return gelu_erf_fast(v); });
-    else
-      ML::template stage_part<P>(lds, acc, [](float v) { return v; });
-    ML::for_each_staged_chunk(lds, [&](int m, int col, u32x4_t v) {
-      const int p = ch.row0 + P * ML::kPartRows + m;
-      const int f = n0 + col;
-      *reinterpret_cast<u32x4_t*>(a.out + ((p / kBS) * ffn_blocks + f / kBS) * (kBS * kBS) + (p % kBS) * kBS +
-                                  (f % kBS)) = v;
-    });
-  });
-}
 
 // Expert tiles of the DSD (defined below): 256 columns, chunks of up to 256
 // rows, 4 waves; for a reduction of F >= 8192, 8 waves (as sb_dsd's
@@ -207,6 +188,13 @@ using SddChunkCfg = std::conditional_t<
                        ChunkCfg<R, kSddBN, kSddWaves, kSddStages>>>;
 static_assert(SddChunkCfg<5>::kLdsAlloc <= 160 * 1024, "LDS");
 
+// Whether a narrow SDD tile of an expert of one row block may stop at its
+// last real 32-row group: when the DSD reads no further, as its 4-wave
+// row-block tiles and its narrow tiles do.
+__device__ __forceinline__ bool sdd_cuts_single(int live_rb, int ffn_dim, int d_model, int cus) {
+  return ffn_dim < kDsdDeepF || narrow_width(live_rb, d_model, kDsdWidestNarrow, cus) > 0;
+}
+
 template <class CfgB>
 __global__ void __launch_bounds__(64 * kSddWaves)
     sdd_layer_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w1,
@@ -220,29 +208,48 @@ __global__ void __launch_bounds__(64 * kSddWaves)
   using CfgH = SddHalfTile;
   static_assert(CfgH::kThreads == CfgB::kThreads && 2 * CfgH::BN == CfgB::BN, "half tiles: same workgroup");
   __shared__ __attribute__((aligned(1024)))
-  uint8_t lds[max_int(max_int(chunk_lds_bytes<kSddBN, kSddWaves, kSddStages, kSddRmax>(),
-                               chunk_lds_bytes<kSddBN, kSddWaves, 4, 4>()),
-                       max_int(CfgB::kLdsAlloc, CfgH::kLdsAlloc))];
+  uint8_t lds[max_int(max_int(max_int(chunk_lds_bytes<kSddBN, kSddWaves, kSddStages, kSddRmax>(),
+                                       chunk_lds_bytes<kSddBN, kSddWaves, 4, 4>()),
+                               max_int(CfgB::kLdsAlloc, CfgH::kLdsAlloc)),
+                       narrow_lds_bytes<kSddWaves, kSddWidestNarrow>())];
   // Workgroups past both tilings' tiles leave before the summary: every
   // chunk starts a row block of its own, so there are at most live row
   // blocks x slices tiles either way, numbered up to kNumXcd - 1 chunk rows
   // past them by the XCD deal, plus the split halves of a short last round.
-  // The counts are loaded alongside padded_offsets[E], ahead of the exit test.
-  const int32_t first = expert_counts(tokens_per_expert, num_experts, 0);
   const int live_rb = __builtin_amdgcn_readfirstlane(padded_offsets[num_experts]) / kBS;
-  if (static_cast<int>(blockIdx.x) >= (live_rb + kNumXcd) * (ffn_dim / kSddBN) + tail_slack) return;
-  const LayoutSummary sum =
-      summarize_layout<kSddRmax, 4, dsd_rmax<4>(), dsd_rmax<8>()>(tokens_per_expert, num_experts, first);
   const SddArgs a{x, w1, row_token, out, num_tokens, d_model, ffn_dim, apply_gelu};
+  const int cus = cus_per_xcd * kNumXcd;
+  int32_t first;
+  LayoutSummary sum;
   // The DSD's own choice (dsd_layer_kernel): its expert tiles when the
   // routing is balanced, F >= kDsdExpertMinF and its grid of dsd_grid
   // workgroups holds them all.
-  const bool dsd_expert =
-      force == 1 || (ffn_dim >= kDsdExpertMinF && expert_stage_runs(sum, num_experts, kGateDsd, force) &&
-                     static_cast<int64_t>(ffn_dim >= kDsdDeepF ? sum.chunks_d : sum.chunks_c) * (d_model / kDsdBN) <=
-                         dsd_grid);
-  if (!(expert_stage_runs(sum, num_experts, kGateSdd, force, ffn_dim / kSddBN, cus_per_xcd * kNumXcd) &&
-        dsd_expert)) {
+  auto expert_choice = [&] {
+    first = expert_counts(tokens_per_expert, num_experts, 0);
+    sum = summarize_layout<kSddRmax, 4, dsd_rmax<4>(), dsd_rmax<8>()>(tokens_per_expert, num_experts, first);
+    const bool dsd_expert =
+        force == 1 || (ffn_dim >= kDsdExpertMinF && expert_stage_runs(sum, num_experts, kGateDsd, force) &&
+                       static_cast<int64_t>(ffn_dim >= kDsdDeepF ? sum.chunks_d : sum.chunks_c) *
+                               (d_model / kDsdBN) <=
+                           dsd_grid);
+    return expert_stage_runs(sum, num_experts, kGateSdd, force, ffn_dim / kSddBN, cus) && dsd_expert;
+  };
+  const int bn = force == 0 ? narrow_width(live_rb, ffn_dim, kSddWidestNarrow, cus) : 0;
+  if (bn > 0) {
+    Chunk ch;
+    int slice;
+    if (!narrow_chunk(static_cast<int>(blockIdx.x), live_rb, ffn_dim / bn, row_block_expert, tokens_per_expert,
+                      padded_offsets, num_experts, max_row_blocks, sdd_cuts_single(live_rb, ffn_dim, d_model, cus),
+                      expert_choice, &ch, &slice))
+      return;
+    with_narrow<kSddWaves, kSddWidestNarrow>(ch.groups, bn, [&](auto cfg) {
+      using Cfg = typename decltype(cfg)::type;
+      sdd_chunk_tile<Cfg>(lds, a, ch, slice * Cfg::BN);
+    });
+    return;
+  }
+  if (static_cast<int>(blockIdx.x) >= (live_rb + kNumXcd) * (ffn_dim / kSddBN) + tail_slack) return;
+  if (!expert_choice()) {
     // Row blocks: the chunks of up to 128 rows are the live row blocks, in
     // order; every row is computed and written (padding rows read as zeros),
     // except past the last 32-row group of an expert of at most 96 rows when
@@ -341,21 +348,39 @@ using SddPairTile = DmaCfg<256, 256, 32, 4, 2, 4, 0, 2, 5, 1, 1>;
 template <class CfgP, class CfgS, class CfgSH>
 __global__ void __launch_bounds__(CfgP::kThreads)
     sdd_pair_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w1,
-                    const int32_t* __restrict__ row_token, const int32_t* __restrict__ tokens_per_expert,
-                    const int32_t* __restrict__ padded_offsets, uint16_t* __restrict__ out, int32_t num_tokens,
-                    int32_t d_model, int32_t ffn_dim, int32_t num_experts, int32_t max_row_blocks,
-                    int32_t apply_gelu, int32_t cus_per_xcd) {
+                    const int32_t* __restrict__ row_token, const int32_t* __restrict__ row_block_expert,
+                    const int32_t* __restrict__ tokens_per_expert, const int32_t* __restrict__ padded_offsets,
+                    uint16_t* __restrict__ out, int32_t num_tokens, int32_t d_model, int32_t ffn_dim,
+                    int32_t num_experts, int32_t max_row_blocks, int32_t apply_gelu, int32_t force,
+                    int32_t cus_per_xcd) {
   static_assert(CfgP::kThreads == CfgS::kThreads && CfgP::BN == CfgS::BN, "one workgroup and slice width");
   static_assert(CfgSH::kThreads == CfgS::kThreads && 2 * CfgSH::BN == CfgS::BN && CfgSH::BK == CfgS::BK,
                 "a single's column halves: same workgroup and K steps");
   static_assert(CfgP::BM == 2 * kBS && CfgS::BM == kBS && CfgSH::BM == kBS, "pairs and singles of row blocks");
-  __shared__ __attribute__((aligned(1024))) uint8_t lds[max_int(CfgP::kLdsAlloc, max_int(CfgS::kLdsAlloc,
-                                                                                         CfgSH::kLdsAlloc))];
+  __shared__ __attribute__((aligned(1024)))
+  uint8_t lds[max_int(max_int(CfgP::kLdsAlloc, narrow_lds_bytes<kSddWaves, kSddWidestNarrow>()),
+                      max_int(CfgS::kLdsAlloc, CfgSH::kLdsAlloc))];
   // Workgroup bid is XCD bid % 8's tile bid / 8 (units x slices, unit-major,
   // a short last round of singles as column halves; pair_tile_for).
-  const int32_t first = expert_counts(tokens_per_expert, num_experts, 0);
   const int live_rb = __builtin_amdgcn_readfirstlane(padded_offsets[num_experts]) / kBS;
   const int slices = ffn_dim / CfgP::BN;
+  const SddArgs a{x, w1, row_token, out, num_tokens, d_model, ffn_dim, apply_gelu};
+  const int bn = force == 0 ? narrow_width(live_rb, ffn_dim, kSddWidestNarrow, cus_per_xcd * kNumXcd) : 0;
+  if (bn > 0) {
+    Chunk nch;
+    int nslice;
+    if (!narrow_chunk(static_cast<int>(blockIdx.x), live_rb, ffn_dim / bn, row_block_expert, tokens_per_expert,
+                      padded_offsets, num_experts, max_row_blocks,
+                      sdd_cuts_single(live_rb, ffn_dim, d_model, cus_per_xcd * kNumXcd), [] { return false; }, &nch,
+                      &nslice))
+      return;
+    with_narrow<kSddWaves, kSddWidestNarrow>(nch.groups, bn, [&](auto cfg) {
+      using Cfg = typename decltype(cfg)::type;
+      sdd_chunk_tile<Cfg>(lds, a, nch, nslice * Cfg::BN);
+    });
+    return;
+  }
+  const int32_t first = expert_counts(tokens_per_expert, num_experts, 0);
   if (static_cast<int>(blockIdx.x) / kNumXcd >= pair_units_per_xcd(live_rb) * slices + cus_per_xcd / 2) return;
   const PairCounts pc = pair_counts(tokens_per_expert, num_experts, first);
   bool single;
@@ -368,7 +393,6 @@ __global__ void __launch_bounds__(CfgP::kThreads)
   if (ch.expert < 0 || ch.expert >= num_experts || ch.row0 < 0 || ch.rows < 1 ||
       ch.row0 + 32 * ch.groups > max_row_blocks * kBS)
     return;
-  const SddArgs a{x, w1, row_token, out, num_tokens, d_model, ffn_dim, apply_gelu};
   if (ch.groups == CfgP::BM / 32) {
     sdd_chunk_tile<CfgP>(lds, a, ch, slice * CfgP::BN);
     return;
@@ -394,73 +418,6 @@ __global__ void __launch_bounds__(CfgP::kThreads)
 
 // ------------------------------------------------------------------ DSD ---
 
-// A: the chunk's rows of H, read in place. All of H is one buffer; lane row
-// j of the chunk sits in row block row0/128 + j/128 at row j % 128, so its
-// offset from the chunk's first block of the K step is fixed per lane, and
-// the step moves the scalar offset (4 steps of 32 per 128-wide block).
-template <class Cfg>
-struct DsdChunkSrc {
-  static constexpr int kStepsPerBlock = kBS / Cfg::BK;
-  __amdgpu_buffer_rsrc_t h_rsrc, w_rsrc;
-  uint32_t h_base;  // byte offset of the chunk's first H block
-  uint32_t w_step_bytes, n0_bytes;
-  uint32_t a_off[Cfg::kAInstr];
-  uint32_t b_off[Cfg::kBInstr];
-  __device__ __forceinline__ uint32_t a_voff(int q) const { return a_off[q]; }
-  __device__ __forceinline__ uint32_t b_voff(int q) const { return b_off[q]; }
-  __device__ __forceinline__ void a_src(int t, __amdgpu_buffer_rsrc_t* r, uint32_t* s) const {
-    *r = h_rsrc;
-    *s = h_base + static_cast<uint32_t>(t / kStepsPerBlock) * (kBS * kBS * 2) +
-         static_cast<uint32_t>(t % kStepsPerBlock) * (Cfg::BK * 2);
-  }
-  __device__ __forceinline__ void b_src(int t, __amdgpu_buffer_rsrc_t* r, uint32_t* s) const {
-    *r = w_rsrc;
-    *s = static_cast<uint32_t>(t) * w_step_bytes + n0_bytes;
-  }
-};
-
-struct DsdArgs {
-  const uint16_t* h;
-  const uint16_t* w2;
-  uint16_t* out;
-  int64_t h_bytes;
-  int32_t ffn_dim, d_model;
-};
-
-template <class Cfg>
-__device__ __forceinline__ void dsd_chunk_tile(uint8_t* __restrict__ lds, const DsdArgs& a, const Chunk& ch, int n0) {
-  using ML = DmaMainloop<Cfg>;
-  const uint32_t ffn_blocks = static_cast<uint32_t>(a.ffn_dim / kBS);
-  DsdChunkSrc<Cfg> src;
-  src.h_rsrc = make_rsrc(a.h, static_cast<uint32_t>(a.h_bytes));
-  src.h_base = static_cast<uint32_t>(ch.row0 / kBS) * ffn_blocks * (kBS * kBS * 2);
-  src.w_rsrc = make_rsrc(a.w2 + static_cast<int64_t>(ch.expert) * a.ffn_dim * a.d_model,
-                         static_cast<uint32_t>(a.ffn_dim) * static_cast<uint32_t>(a.d_model) * 2u);
-  src.w_step_bytes = static_cast<uint32_t>(Cfg::BK) * static_cast<uint32_t>(a.d_model) * 2u;
-  src.n0_bytes = static_cast<uint32_t>(n0) * 2u;
-  const ADmaPos<Cfg> ap;
-#pragma unroll
-  for (int q = 0; q < Cfg::kAInstr; ++q) {
-    const uint32_t j = static_cast<uint32_t>(ap.row[q]);
-    src.a_off[q] = static_cast<int>(j) < ch.rows
-                       ? ((j / kBS) * ffn_blocks * (kBS * kBS) + (j % kBS) * kBS) * 2u + ap.chunk[q] * 16u
-                       : kOutOfRange;
-  }
-  const BDmaPos<Cfg> bp;
-#pragma unroll
-  for (int q = 0; q < Cfg::kBInstr; ++q)
-    src.b_off[q] = (static_cast<uint32_t>(bp.row[q]) * a.d_model + bp.col[q]) * 2u;
-
-  typename ML::Acc acc;
-  ML::run(lds, src, a.ffn_dim / Cfg::BK, acc);
-
-  ML::stage_tile(lds, acc, [](float v) { return v; });
-  uint16_t* out_tile = a.out + static_cast<int64_t>(ch.row0) * a.d_model + n0;
-  ML::for_each_staged_chunk(lds, [&](int m, int col, u32x4_t v) {
-    if (m < ch.rows) *reinterpret_cast<u32x4_t*>(out_tile + static_cast<int64_t>(m) * a.d_model + col) = v;
-  });
-}
-
 // Expert tiles of the DSD: 4 waves, 256 columns, chunks of up to 256 rows.
 // Row-block tiles: 4 waves, 128 x CfgB::BN, every row of the row block read
 // and written, as sb_dsd's default tile does, except for an expert of one
@@ -481,20 +438,38 @@ __global__ void __launch_bounds__(64 * WAVES)
   using CfgH = DsdCfg<4, CfgB::BN / 2, WAVES, kDsdStages>;
   constexpr int kRmax = dsd_rmax<WAVES>();
   __shared__ __attribute__((aligned(1024)))
-  uint8_t lds[max_int(chunk_lds_bytes<kDsdBN, WAVES, kDsdStages, kRmax>(), max_int(CfgB::kLdsAlloc, CfgH::kLdsAlloc))];
-  // As in the SDD: at most live row blocks x D/256 tiles either way, plus
-  // the split halves of a short last round.
-  const int32_t first = expert_counts(tokens_per_expert, num_experts, 0);
+  uint8_t lds[max_int(max_int(chunk_lds_bytes<kDsdBN, WAVES, kDsdStages, kRmax>(), narrow_lds_bytes<WAVES, kDsdWidestNarrow>()),
+                      max_int(CfgB::kLdsAlloc, CfgH::kLdsAlloc))];
   const int live_rb = __builtin_amdgcn_readfirstlane(padded_offsets[num_experts]) / kBS;
-  if (static_cast<int>(blockIdx.x) >= live_rb * (d_model / kDsdBN) + tail_slack) return;
-  const LayoutSummary sum = summarize_layout<kRmax, 4>(tokens_per_expert, num_experts, first);
   const DsdArgs a{h, w2, out, h_bytes, ffn_dim, d_model};
+  int32_t first;
+  LayoutSummary sum;
   // Expert tiles for balanced routing over a reduction of at least
   // kDsdExpertMinF. The grid may hold fewer workgroups than expert tiles
   // (see the launch): then the row blocks take the stage.
-  const bool fits = static_cast<int64_t>(sum.chunks_a) * (d_model / kDsdBN) <= static_cast<int64_t>(tile_grid);
-  const bool chosen = ffn_dim >= kDsdExpertMinF && expert_stage_runs(sum, num_experts, kGateDsd, force) && fits;
-  if (!(chosen || force == 1)) {
+  auto expert_choice = [&] {
+    first = expert_counts(tokens_per_expert, num_experts, 0);
+    sum = summarize_layout<kRmax, 4>(tokens_per_expert, num_experts, first);
+    const bool fits = static_cast<int64_t>(sum.chunks_a) * (d_model / kDsdBN) <= static_cast<int64_t>(tile_grid);
+    return force == 1 || (ffn_dim >= kDsdExpertMinF && expert_stage_runs(sum, num_experts, kGateDsd, force) && fits);
+  };
+  const int bn = force == 0 ? narrow_width(live_rb, d_model, kDsdWidestNarrow, cus_per_xcd * kNumXcd) : 0;
+  if (bn > 0) {
+    Chunk ch;
+    int slice;
+    if (!narrow_chunk(static_cast<int>(blockIdx.x), live_rb, d_model / bn, row_block_expert, tokens_per_expert,
+                      padded_offsets, num_experts, max_row_blocks, true, expert_choice, &ch, &slice))
+      return;
+    with_narrow<WAVES, kDsdWidestNarrow>(ch.groups, bn, [&](auto cfg) {
+      using Cfg = typename decltype(cfg)::type;
+      dsd_chunk_tile<Cfg>(lds, a, ch, slice * Cfg::BN);
+    });
+    return;
+  }
+  // As in the SDD: at most live row blocks x D/256 tiles either way, plus
+  // the split halves of a short last round.
+  if (static_cast<int>(blockIdx.x) >= live_rb * (d_model / kDsdBN) + tail_slack) return;
+  if (!expert_choice()) {
     // Row blocks: the chunks of up to 128 rows are the live row blocks, in order.
     // The tiles of a short last round run as column halves (split_tail).
     const int blocks = sum.chunks_b;
@@ -635,7 +610,7 @@ int launch_sdd_layer(const void* x, const void* w1, const int32_t* row_token, co
   int cus = 0;
   if (const int rc = device_cus(&cus)) return rc;
   const int64_t slack = split_tail_slack(cus) + kNumXcd * (ffn_dim / kSddBN);
-  sdd_layer_kernel<CfgB><<<static_cast<uint32_t>(tiles + slack), 64 * kSddWaves, 0, stream>>>(
+  sdd_layer_kernel<CfgB><<<static_cast<uint32_t>(std::max<int64_t>(tiles + slack, cus)), 64 * kSddWaves, 0, stream>>>(
       static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w1), row_token, row_block_expert, row_offsets,
       tokens_per_expert, padded_offsets, static_cast<uint16_t*>(out), static_cast<int32_t>(num_tokens),
       static_cast<int32_t>(d_model), static_cast<int32_t>(ffn_dim), static_cast<int32_t>(num_experts),
@@ -658,9 +633,10 @@ int dispatch_sdd_layer(const void* x, const void* w1, const int32_t* row_token, 
                                        apply_gelu, force, stream);
 }
 
-int launch_sdd_pairs(const void* x, const void* w1, const int32_t* row_token, const int32_t* tokens_per_expert,
-                     const int32_t* padded_offsets, void* out, int64_t num_tokens, int64_t d_model, int64_t ffn_dim,
-                     int64_t num_experts, int64_t max_row_blocks, int32_t apply_gelu, hipStream_t stream) {
+int launch_sdd_pairs(const void* x, const void* w1, const int32_t* row_token, const int32_t* row_block_expert,
+                     const int32_t* tokens_per_expert, const int32_t* padded_offsets, void* out, int64_t num_tokens,
+                     int64_t d_model, int64_t ffn_dim, int64_t num_experts, int64_t max_row_blocks, int32_t apply_gelu,
+                     int32_t force, hipStream_t stream) {
   if (!reduction_fits<SddPairTile>(d_model) || !reduction_fits<SddNarrowTile>(d_model) ||
       !reduction_fits<SddNarrowHalfTile>(d_model))
     return fail(SB_ERR_INVALID, "sdd_experts: D (%lld) is not a whole number of the tiles' K steps",
@@ -674,11 +650,11 @@ int launch_sdd_pairs(const void* x, const void* w1, const int32_t* row_token, co
       int64_t{kNumXcd} *
       (int64_t{pair_units_per_xcd(static_cast<int>(max_row_blocks))} * (ffn_dim / SddPairTile::BN) + cus_per_xcd / 2);
   sdd_pair_kernel<SddPairTile, SddNarrowTile, SddNarrowHalfTile>
-      <<<static_cast<uint32_t>(grid), SddPairTile::kThreads, 0, stream>>>(
-          static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w1), row_token, tokens_per_expert,
-          padded_offsets, static_cast<uint16_t*>(out), static_cast<int32_t>(num_tokens),
+      <<<static_cast<uint32_t>(std::max<int64_t>(grid, cus)), SddPairTile::kThreads, 0, stream>>>(
+          static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w1), row_token, row_block_expert,
+          tokens_per_expert, padded_offsets, static_cast<uint16_t*>(out), static_cast<int32_t>(num_tokens),
           static_cast<int32_t>(d_model), static_cast<int32_t>(ffn_dim), static_cast<int32_t>(num_experts),
-          static_cast<int32_t>(max_row_blocks), apply_gelu, cus_per_xcd);
+          static_cast<int32_t>(max_row_blocks), apply_gelu, force, cus_per_xcd);
   return check_launch("sdd_experts");
 }
 
@@ -696,7 +672,7 @@ int launch_dsd_layer(const void* h, const void* w2, const int32_t* tokens_per_ex
   int cus = 0;
   if (const int rc = device_cus(&cus)) return rc;
   const int64_t slack = split_tail_slack(cus);
-  dsd_layer_kernel<CfgB, WAVES><<<static_cast<uint32_t>(tiles + slack), 64 * WAVES, 0, stream>>>(
+  dsd_layer_kernel<CfgB, WAVES><<<static_cast<uint32_t>(std::max<int64_t>(tiles + slack, cus)), 64 * WAVES, 0, stream>>>(
       static_cast<const uint16_t*>(h), static_cast<const uint16_t*>(w2), tokens_per_expert, padded_offsets,
       row_block_expert, static_cast<uint16_t*>(out), h_bytes, static_cast<int32_t>(num_experts),
       static_cast<int32_t>(ffn_dim), static_cast<int32_t>(d_model), static_cast<int32_t>(max_row_blocks),
@@ -742,8 +718,9 @@ extern "C" int sb_sdd_experts(const void* x, const void* w1, const int32_t* row_
     return sb_sdd(x, w1, row_token, row_block_expert, row_offsets, out, num_tokens, d_model, ffn_dim, num_experts,
                   max_row_blocks, apply_gelu, stream);
   if (ffn_dim % kSddBN != 0) {
-    const int rc = launch_sdd_pairs(x, w1, row_token, tokens_per_expert, padded_offsets, out, num_tokens, d_model,
-                                    ffn_dim, num_experts, max_row_blocks, apply_gelu, as_stream(stream));
+    const int rc = launch_sdd_pairs(x, w1, row_token, row_block_expert, tokens_per_expert, padded_offsets, out,
+                                    num_tokens, d_model, ffn_dim, num_experts, max_row_blocks, apply_gelu, force,
+                                    as_stream(stream));
     return rc ? rc : clear_ok();
   }
   const int rc = dispatch_sdd_layer(x, w1, row_token, row_block_expert, row_offsets, tokens_per_expert, padded_offsets,

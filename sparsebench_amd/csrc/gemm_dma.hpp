@@ -93,8 +93,11 @@ __device__ __forceinline__ void wait_vmcnt() {
 // B in slot t % BSTAGES, loaded BSTAGES-1 steps ahead (DmaMainloop::
 // run_split_xs). For tall tiles whose A area leaves no room for a fourth
 // whole stage: the weight stream, whose misses go to HBM, keeps its lead.
+// XW: waves of the workgroup past the WM x WN that compute (PIPE 5,
+// unpaired): they issue their share of the loads and keep the barriers, for
+// tiles narrower than their kernel's workgroup.
 template <int BM_, int BN_, int BK_, int STAGES_, int WM_ = 2, int WN_ = 2, int CPA_ = 0, int CPB_ = 0, int PIPE_ = 0,
-          int EPI_PARTS_ = 1, int APAIR_ = 0, int BSTAGES_ = 0>
+          int EPI_PARTS_ = 1, int APAIR_ = 0, int BSTAGES_ = 0, int XW_ = 0>
 struct DmaCfg {
   static constexpr int BM = BM_, BN = BN_, BK = BK_, STAGES = STAGES_;
   static constexpr int BSTAGES = BSTAGES_ > 0 ? BSTAGES_ : STAGES_;
@@ -104,7 +107,8 @@ struct DmaCfg {
   static constexpr int EPI_PARTS = EPI_PARTS_;
   static constexpr bool APAIR = APAIR_ != 0;
   static constexpr int WM = WM_, WN = WN_;
-  static constexpr int kWaves = WM * WN;
+  static constexpr int kComputeWaves = WM * WN;
+  static constexpr int kWaves = kComputeWaves + XW_;
   static constexpr int kThreads = 64 * kWaves;
   static constexpr int WTM = BM / WM, WTN = BN / WN;
   static constexpr int TM = WTM / 32, TN = WTN / 32;
@@ -140,11 +144,12 @@ struct DmaCfg {
   static_assert(kBRowBytes <= 1024, "one DMA row per instruction at most");
   static constexpr int kBChunksPerRow = BN / 8;
   static_assert(BK == 32 || BK == 64, "BK");
-  static_assert(BN == 128 || BN == 256 || BN == 512, "BN");
+  static_assert(XW_ == 0 || (PIPE == 5 && !APAIR && !SPLIT), "load-only waves: run_xs");
+  static_assert(BN == 64 || BN == 128 || BN == 256 || BN == 512, "BN");
   static_assert(WTM % 32 == 0 && WTN % 32 == 0, "waves own whole 32 x 32 blocks");
   static_assert(kAInstr >= 1 && kABytes >= BM * kARowBytes, "the A area holds BM rows");
   static_assert(kBInstr >= 1 && kBInstr * kWaves * 1024 == kBBytes, "B step splits into whole 1 KB DMA rows");
-  static_assert(STAGES >= 2 && STAGES <= 8, "STAGES");
+  static_assert(STAGES >= 2 && STAGES <= 16, "STAGES");
   static_assert(kLdsAlloc <= 160 * 1024, "LDS");
   static_assert((APAIR ? kLaterLoadsOdd : kLaterLoads) <= 63, "vmcnt");
   static_assert(!APAIR || (BK == 32 && (STAGES == 3 || STAGES == 4) && (PIPE == 3 || PIPE == 4 || PIPE == 5)),
@@ -176,6 +181,15 @@ __device__ __forceinline__ int swz_a(int r) {
   else return (r >> 2) & 3;                             // 4 rows per 256 B
 }
 
+// B rows are BN/8 16-byte chunks; a 32-column block is 4 of them (64 bytes).
+// Block b of row k sits at b ^ swz_b(k): the 8 rows x 64 bytes of one
+// transposing read (k0 .. k0+3 and k0+8 .. k0+11) then hit each quarter of
+// the 256-byte bank span twice, for rows of 256 bytes or more and of 128.
+template <int BN>
+__device__ __forceinline__ int swz_b(int k) {
+  return BN >= 128 ? k & 3 : (k >> 1) & 1;
+}
+
 // This lane's LDS row / chunk for A DMA instruction q, and the logical
 // chunk it must fetch.
 template <class Cfg>
@@ -202,7 +216,7 @@ struct BDmaPos {
     for (int q = 0; q < Cfg::kBInstr; ++q) {
       row[q] = Cfg::kBRowsPerInstr * (Cfg::kBInstr * wave + q) + lane / Cfg::kBChunksPerRow;
       const int p = lane % Cfg::kBChunksPerRow;
-      col[q] = 8 * (p ^ (4 * (row[q] & 3)));
+      col[q] = 8 * (p ^ (4 * swz_b<Cfg::BN>(row[q])));
     }
   }
 };
@@ -402,7 +416,7 @@ struct DmaMainloop {
 #pragma unroll
       for (int jn = 0; jn < Cfg::TN; ++jn) {
         const int blk = (wn * Cfg::WTN) / 32 + jn;  // 32-column block index
-        const int chunk = 4 * (blk ^ (jj >> 2)) + 2 * (g & 1) + ((jj & 3) >> 1);
+        const int chunk = 4 * (blk ^ swz_b<Cfg::BN>(krow)) + 2 * (g & 1) + ((jj & 3) >> 1);
         b_off[jn] = krow * Cfg::kBRowBytes + chunk * 16 + (jj & 1) * 8;
       }
     }
@@ -698,6 +712,37 @@ struct DmaMainloop {
     compute_xs<false>(a_slot(lds, t), b_slot(lds, t), 0, acc, NoDma{}, fr, a, b, nullptr, nullptr, 0, NoWait{});
   }
 
+  // Whether this wave computes (all do but the XW load-only ones).
+  __device__ __forceinline__ static bool computes() {
+    if constexpr (Cfg::kWaves == Cfg::kComputeWaves) return true;
+    else return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) < Cfg::kComputeWaves;
+  }
+
+  // The loads, waits and barriers of run_xs alone, for a load-only wave:
+  // its step t issues step t+STAGES-1's share into the slot that the
+  // computing waves read to its end before the barrier at the end of step
+  // t-1, then waits for its share of step t+1 and meets them there.
+  template <class Src>
+  __device__ __forceinline__ static void run_loads(uint8_t* lds, const Src& src, int n) {
+    constexpr int S = Cfg::STAGES;
+    issue_b_first(step_dma(lds, 0, src));
+#pragma unroll
+    for (int s = 1; s < S - 1; ++s)
+      if (s < n) issue_all(step_dma(lds, s, src));
+    wait_steps<Cfg::kLoadsPerStep, S - 2>(n - 1);
+    __builtin_amdgcn_s_barrier();
+    int t = 0;
+    for (; t + S - 1 < n; ++t) {
+      issue_all(step_dma(lds, t + S - 1, src));
+      wait_vmcnt<Cfg::kLaterLoads>();
+      __builtin_amdgcn_s_barrier();
+    }
+    for (; t + 1 < n; ++t) {
+      wait_steps<Cfg::kLoadsPerStep, S - 2>(n - 2 - t);
+      __builtin_amdgcn_s_barrier();
+    }
+  }
+
   // PIPE 5, unpaired.
   template <class Src>
   __device__ __forceinline__ static void run_xs(uint8_t* lds, const Src& src, int n, Acc& acc) {
@@ -783,7 +828,8 @@ struct DmaMainloop {
     if constexpr (Cfg::PIPE == 5) {
       if constexpr (Cfg::APAIR) run_paired_xs(lds, src, num_steps, acc);
       else if constexpr (Cfg::SPLIT) run_split_xs(lds, src, num_steps, acc);
-      else run_xs(lds, src, num_steps, acc);
+      else if (computes()) run_xs(lds, src, num_steps, acc);
+      else run_loads(lds, src, num_steps);
       return;
     }
     if constexpr (Cfg::APAIR) {
@@ -836,10 +882,10 @@ struct DmaMainloop {
   static_assert(kStagedBytes <= Cfg::kLdsAlloc, "staged tile fits the kernel's LDS");
   static constexpr int kPartGroups = Cfg::TM / Cfg::EPI_PARTS;  // 32-row groups per part (WM == 1 when split)
   static constexpr int kPartRows = Cfg::BM / Cfg::EPI_PARTS;
-  static_assert(Cfg::BN >= 128, "16 chunks per row at least");
+  static constexpr int kStagedSwz = Cfg::BN >= 128 ? 15 : Cfg::BN / 8 - 1;  // within a row's chunks
 
   __device__ __forceinline__ static int staged_offset(int r, int chunk) {
-    return r * (Cfg::BN * 2) + ((chunk ^ (r & 15)) << 4);
+    return r * (Cfg::BN * 2) + ((chunk ^ (r & kStagedSwz)) << 4);
   }
 
   template <class Fn>
@@ -853,21 +899,23 @@ struct DmaMainloop {
   template <int P, class Fn>
   __device__ __forceinline__ static void stage_part(uint8_t* __restrict__ lds, Acc& acc, Fn fn) {
     __syncthreads();  // every wave is done reading the ring (or the previous part)
+    if (computes()) {
 #pragma unroll
-    for (int jn = 0; jn < Cfg::TN; ++jn)
+      for (int jn = 0; jn < Cfg::TN; ++jn)
 #pragma unroll
-      for (int i = P * kPartGroups; i < (P + 1) * kPartGroups; ++i) {
-        const int m = out_row(i) - P * kPartRows;
+        for (int i = P * kPartGroups; i < (P + 1) * kPartGroups; ++i) {
+          const int m = out_row(i) - P * kPartRows;
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const int n = out_col(jn, g);
-          float v[4];
+          for (int g = 0; g < 4; ++g) {
+            const int n = out_col(jn, g);
+            float v[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = fn(acc[jn][i][4 * g + e]);
-          *reinterpret_cast<u32x2_t*>(lds + staged_offset(m, n >> 3) + (n & 7) * 2) =
-              u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+            for (int e = 0; e < 4; ++e) v[e] = fn(acc[jn][i][4 * g + e]);
+            *reinterpret_cast<u32x2_t*>(lds + staged_offset(m, n >> 3) + (n & 7) * 2) =
+                u32x2_t{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+          }
         }
-      }
+    }
     __syncthreads();
   }
 
@@ -877,10 +925,10 @@ struct DmaMainloop {
   __device__ __forceinline__ static void for_each_staged_chunk(const uint8_t* __restrict__ lds, Fn fn) {
     constexpr int kChunksPerRow = Cfg::BN / 8;
     constexpr int kChunks = kPartRows * kChunksPerRow;
-    static_assert(kChunks % Cfg::kThreads == 0, "whole passes");
 #pragma unroll
     for (int q0 = 0; q0 < kChunks; q0 += Cfg::kThreads) {
       const int q = q0 + static_cast<int>(threadIdx.x);
+      if (kChunks % Cfg::kThreads != 0 && q >= kChunks) break;
       const int r = q / kChunksPerRow, c = q % kChunksPerRow;
       fn(r, c * 8, *reinterpret_cast<const u32x4_t*>(lds + staged_offset(r, c)));
     }

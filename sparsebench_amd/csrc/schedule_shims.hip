@@ -2,7 +2,7 @@
 // over the same __host__ __device__ functions the kernels call
 // (common.hpp: xcd_remap, split_tail, split_tail_slack, tile_coords;
 // expert_chunks.hpp: balanced_chunk_tile, lpt_group_tile, pair_units_per_xcd,
-// pair_tile_for), so tests/test_tile_schedules.py checks the compiled
+// pair_tile_for, narrow_width, narrow_tile_for), so tests/test_tile_schedules.py checks the compiled
 // mappings themselves. Part of the tool library (libsparsebench_probe.so),
 // not of libsparsebench_hip.so's C ABI. No kernel runs.
 
@@ -40,4 +40,12 @@ extern "C" int sbt_pair_tile_for(int bid, int pairs, int singles, int slices, in
 
 extern "C" void sbt_lpt_group_tile(int local, int groups, int slices, uint32_t big, int* pos, int* slice) {
   lpt_group_tile(local, groups, slices, big, pos, slice);
+}
+
+extern "C" int sbt_narrow_width(int live_rb, int columns, int widest, int cus) {
+  return narrow_width(live_rb, columns, widest, cus);
+}
+
+extern "C" void sbt_narrow_tile_for(int bid, int live_rb, int slices, int* rb, int* slice) {
+  narrow_tile_for(bid, live_rb, slices, rb, slice);
 }
