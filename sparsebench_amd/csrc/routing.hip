@@ -9,16 +9,17 @@
 // Launches, all on the caller's stream:
 //   1. count    one workgroup per chunk of 1024 copies: per-expert counts of
 //               the chunk, plus a count of bad ids in column E.
-//   2. offsets  (only beyond kScanChunks chunks) one workgroup: exclusive
+//   2. columns  (only beyond kScanChunks chunks) a few workgroups: exclusive
 //               prefix of every expert's column over the chunks (in place),
-//               tokens_per_expert, padded_offsets, error.
+//               tokens_per_expert, error.
 //   3. place    first C workgroups: each copy's row, ranked inside its wave
 //               by ballot bit-slicing (no atomics, so the order is stable);
 //               the remaining workgroups write row_offsets / col_indices /
-//               row_block_expert and mark every non-copy row -1. Up to
-//               kScanChunks chunks, every workgroup first sums the columns
-//               of the counts itself (route_place_scan_kernel), in place of
-//               step 2.
+//               row_block_expert and mark every non-copy row -1. Every
+//               workgroup scans the padded sizes itself, from
+//               tokens_per_expert, or up to kScanChunks chunks from the
+//               counts, whose columns it then sums too
+//               (route_place_scan_kernel), in place of step 2.
 // Place's two roles touch disjoint memory and depend only on steps 1-2.
 
 #include <mutex>
@@ -138,46 +139,54 @@ __device__ __forceinline__ int64_t block_inclusive_scan(int64_t v, int64_t* wave
   return v + (wave > 0 ? wave_sums[wave - 1] : 0);
 }
 
-__global__ void __launch_bounds__(kChunk) route_offsets_kernel(int32_t* __restrict__ counts, int32_t num_chunks,
-                                                               int32_t num_experts, int32_t block_size,
+// Columns of the counts, kColumns to a workgroup: column col (copies of
+// expert col, or bad ids for col == E, in each chunk) is replaced in place by
+// the copies in all earlier chunks. Each column's chunks are split into
+// kColumnGroups runs, one a lane: the lanes sum their runs, scan the sums
+// and walk their runs again. Bound by the latency of a few dependent loads:
+// one lane a column, in one workgroup, took 37.9 us at 512 chunks x 256
+// experts (a chain of 128 loads); this takes 4.7 us.
+constexpr int kColumns = 8;  // 32-byte row pieces
+constexpr int kColumnGroups = kChunk / kColumns;
+
+__global__ void __launch_bounds__(kChunk) route_columns_kernel(int32_t* __restrict__ counts, int32_t num_chunks,
+                                                               int32_t num_experts,
                                                                int32_t* __restrict__ tokens_per_expert,
-                                                               int32_t* __restrict__ padded_offsets,
                                                                int32_t* __restrict__ error) {
-  __shared__ int64_t wave_sums[kWaves];
-  const int tid = threadIdx.x;
+  __shared__ int32_t wave_sums[kWaves][kColumns];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int sub = tid % kColumns, group = tid / kColumns;
+  const int col = static_cast<int>(blockIdx.x) * kColumns + sub;
   const int64_t stride = num_experts + 1;
-  int64_t padded = 0;
-  // Column col: copies of expert col (or bad ids, col == E) in each chunk,
-  // replaced in place by the copies in all earlier chunks. The loads do not
-  // depend on each other, so the unrolled walk keeps several in flight.
-  for (int col = tid; col <= num_experts; col += kChunk) {
-    int32_t total = 0;
-    int32_t b = 0;
-    for (; b + 4 <= num_chunks; b += 4) {
-      int32_t* p = counts + b * stride + col;
-      const int32_t c0 = p[0], c1 = p[stride], c2 = p[2 * stride], c3 = p[3 * stride];
-      p[0] = total;
-      p[stride] = total + c0;
-      p[2 * stride] = total + c0 + c1;
-      p[3 * stride] = total + c0 + c1 + c2;
-      total += c0 + c1 + c2 + c3;
-    }
-    for (; b < num_chunks; ++b) {
-      int32_t* p = counts + b * stride + col;
-      const int32_t c0 = *p;
-      *p = total;
-      total += c0;
-    }
-    if (col < num_experts) {
-      tokens_per_expert[col] = total;
-      padded = (static_cast<int64_t>(total) + block_size - 1) / block_size * block_size;
-    } else {
-      error[0] = total > 0 ? 1 : 0;
-    }
+  const int32_t per = (num_chunks + kColumnGroups - 1) / kColumnGroups;
+  const int32_t first = min(group * static_cast<int64_t>(per), static_cast<int64_t>(num_chunks));
+  const int32_t last = min(first + per, num_chunks);
+  const bool live = col <= num_experts;
+  int32_t own = 0;
+  if (live)
+#pragma unroll 4
+    for (int32_t b = first; b < last; ++b) own += counts[b * stride + col];
+  // Inclusive scan over the groups: 8 to a wave, kColumns lanes apart.
+  int32_t incl = own;
+  for (int d = kColumns; d < 64; d <<= 1) {
+    const int32_t below = __shfl_up(incl, d, 64);
+    if (lane >= d) incl += below;
   }
-  const int64_t incl = block_inclusive_scan(tid < num_experts ? padded : 0, wave_sums);
-  if (tid < num_experts) padded_offsets[tid + 1] = static_cast<int32_t>(incl);
-  if (tid == 0) padded_offsets[0] = 0;
+  if (lane >= 64 - kColumns) wave_sums[wave][sub] = incl;
+  __syncthreads();
+  for (int w = 0; w < wave; ++w) incl += wave_sums[w][sub];
+  if (!live) return;
+  int32_t run = incl - own;
+#pragma unroll 4
+  for (int32_t b = first; b < last; ++b) {
+    const int32_t c = counts[b * stride + col];
+    counts[b * stride + col] = run;
+    run += c;
+  }
+  if (group == kColumnGroups - 1) {
+    if (col < num_experts) tokens_per_expert[col] = incl;
+    else error[0] = incl > 0 ? 1 : 0;
+  }
 }
 
 template <typename Idx, typename Tok>
@@ -186,37 +195,48 @@ __global__ void __launch_bounds__(kChunk)
                        int32_t num_bits,
                        const int32_t* __restrict__ valid_tokens, int32_t num_chunks,
                        const int32_t* __restrict__ chunk_base, const int32_t* __restrict__ tokens_per_expert,
-                       const int32_t* __restrict__ padded_offsets, int32_t block_size, int32_t ffn_blocks,
+                       int32_t* __restrict__ padded_offsets, int32_t block_size, int32_t ffn_blocks,
                        int32_t max_row_blocks, int64_t max_rows, int32_t* __restrict__ copy_row,
                        int32_t* __restrict__ row_token, int32_t* __restrict__ row_block_expert,
                        int32_t* __restrict__ row_offsets, int32_t* __restrict__ col_indices) {
-  __shared__ int32_t lds[kWaves * kMaxExperts];  // place: per-wave counts; layout: offsets + counts
+  __shared__ int32_t total[kMaxExperts];
+  __shared__ int32_t offs[kMaxExperts + 1];
+  __shared__ int32_t wave_counts[kWaves * kMaxExperts];
+  __shared__ int64_t wave_sums[kWaves];
   const int tid = threadIdx.x;
+  const bool placing = static_cast<int32_t>(blockIdx.x) < num_chunks;
+  // The copy's loads wait alongside the counts'.
+  const int64_t c = static_cast<int64_t>(blockIdx.x) * kChunk + tid;
+  bool bad = false;
+  int32_t token = -1;
+  const int32_t e = placing ? read_expert(idx, c, n, tokens, num_experts, valid_tokens, &bad, &token) : -1;
+  const int32_t base =
+      e >= 0 ? chunk_base[static_cast<int64_t>(blockIdx.x) * (num_experts + 1) + e] : 0;  // copies of e in earlier chunks
+  const int32_t mine = tid < num_experts ? tokens_per_expert[tid] : 0;
+  if (tid < num_experts) total[tid] = mine;
+  if (placing)
+    for (int i = tid; i < kWaves * num_experts; i += kChunk) wave_counts[i] = 0;
+  const int64_t padded = (static_cast<int64_t>(mine) + block_size - 1) / block_size * block_size;
+  const int64_t incl = block_inclusive_scan(padded, wave_sums);  // synchronizes the workgroup
+  if (tid < num_experts) offs[tid + 1] = static_cast<int32_t>(incl);
+  if (tid == 0) offs[0] = 0;
+  if (blockIdx.x == 0) {
+    if (tid < num_experts) padded_offsets[tid + 1] = static_cast<int32_t>(incl);
+    if (tid == 0) padded_offsets[0] = 0;
+  }
 
-  if (static_cast<int32_t>(blockIdx.x) < num_chunks) {
+  if (placing) {
     // ---- place: copy -> row, stable inside each expert ----
-    const int lane = tid & 63;
     const int wave = tid >> 6;
-    for (int i = tid; i < kWaves * num_experts; i += kChunk) lds[i] = 0;
-    __syncthreads();
-
-    const int64_t c = static_cast<int64_t>(blockIdx.x) * kChunk + tid;
-    bool bad;
-    int32_t token;
-    const int32_t e = read_expert(idx, c, n, tokens, num_experts, valid_tokens, &bad, &token);
     const bool valid = e >= 0;
     const uint64_t peers = same_expert_lanes(valid, e, num_bits);
     const uint64_t lower = peers & lanes_below();
-    if (valid && lower == 0) lds[wave * num_experts + e] = __popcll(peers);  // one writer per (wave, e)
+    if (valid && lower == 0) wave_counts[wave * num_experts + e] = __popcll(peers);  // one writer per (wave, e)
     __syncthreads();
-    (void)lane;
-
     if (valid) {
       int32_t before = 0;
-      for (int w = 0; w < wave; ++w) before += lds[w * num_experts + e];
-      const int32_t row = padded_offsets[e] +
-                          chunk_base[static_cast<int64_t>(blockIdx.x) * (num_experts + 1) + e] + before +
-                          __popcll(lower);
+      for (int w = 0; w < wave; ++w) before += wave_counts[w * num_experts + e];
+      const int32_t row = offs[e] + base + before + __popcll(lower);
       copy_row[c] = row;
       row_token[row] = token;
     } else if (c < n) {
@@ -226,13 +246,9 @@ __global__ void __launch_bounds__(kChunk)
   }
 
   // ---- layout: BSR arrays and the -1 marks of non-copy rows ----
-  int32_t* offs = lds;                    // [E+1] padded_offsets
-  int32_t* cnts = lds + kMaxExperts + 1;  // [E] tokens_per_expert (E <= 1024, fits the array)
-  for (int e = tid; e <= num_experts; e += kChunk) offs[e] = padded_offsets[e];
-  for (int e = tid; e < num_experts; e += kChunk) cnts[e] = tokens_per_expert[e];
   __syncthreads();
   const int64_t i = static_cast<int64_t>(blockIdx.x - num_chunks) * kLayoutItemsPerGroup + tid;
-  layout_item(i, offs, cnts, num_experts, block_size, ffn_blocks, max_row_blocks, max_rows, row_token,
+  layout_item(i, offs, total, num_experts, block_size, ffn_blocks, max_row_blocks, max_rows, row_token,
               row_block_expert, row_offsets, col_indices);
 }
 
@@ -240,7 +256,7 @@ __global__ void __launch_bounds__(kChunk)
 // kernel's per-chunk counts: each workgroup sums every expert's column
 // itself (one lane per expert; num_chunks loads each), over the chunks
 // before its own and over all of them, and scans the padded sizes in LDS.
-// That replaces the one-workgroup offsets kernel and its launch. Workgroup 0
+// That replaces the columns kernel and its launch. Workgroup 0
 // also writes tokens_per_expert, padded_offsets and the error flag. The
 // rest is route_place_kernel's placement and layout.
 constexpr int kScanChunks = 32;
@@ -367,7 +383,7 @@ namespace sb {
 namespace {
 
 // Routing of n copies whose tokens come from `tokens`: count, then place with
-// the offsets scan inside for at most kScanChunks chunks; count, offsets and
+// the column sums inside for at most kScanChunks chunks; count, columns and
 // place beyond.
 template <typename Idx, typename Tok>
 int launch_routing(const Idx* idx, int64_t n, TokenSource<Tok> tokens, int32_t num_experts, int32_t ffn_dim,
@@ -392,9 +408,10 @@ int launch_routing(const Idx* idx, int64_t n, TokenSource<Tok> tokens, int32_t n
         row_block_expert, row_offsets, col_indices);
     return check_launch("routing place");
   }
-  route_offsets_kernel<<<1, kChunk, 0, stream>>>(workspace, num_chunks, num_experts, block_size, tokens_per_expert,
-                                                 padded_offsets, error);
-  if (int rc = check_launch("routing offsets")) return rc;
+  const uint32_t column_groups = static_cast<uint32_t>((num_experts + kColumns) / kColumns);  // columns 0 .. E
+  route_columns_kernel<<<column_groups, kChunk, 0, stream>>>(workspace, num_chunks, num_experts, tokens_per_expert,
+                                                             error);
+  if (int rc = check_launch("routing columns")) return rc;
   route_place_kernel<Idx, Tok><<<num_chunks + layout_groups, kChunk, 0, stream>>>(
       idx, n, tokens, num_experts, num_bits, valid_tokens, num_chunks, workspace, tokens_per_expert, padded_offsets,
       block_size, ffn_blocks, static_cast<int32_t>(max_row_blocks), max_rows, copy_row, row_token, row_block_expert,
@@ -476,7 +493,7 @@ extern "C" int sb_routing_assigned(const void* expert_of_copy, int32_t expert_is
 // kernels.
 //
 // Nothing in it has to start at zero: the count kernel writes every entry
-// of the chunks it covers before the offsets kernel reads it. Calls that
+// of the chunks it covers before a later kernel reads it. Calls that
 // overlap on one GPU (two streams, or a graph replay beside an eager call)
 // share the array and race.
 
