@@ -184,7 +184,7 @@ int sb_routing_assigned(const void* expert_of_copy, int32_t expert_is_i64, const
  * token_offsets[T+1] and token_copies[N]: the copies of token t are
  * token_copies[token_offsets[t] .. token_offsets[t+1]), in ascending copy
  * order; copies with copy_row < 0 are left out and the unused tail of
- * token_copies is -1. One workgroup; deterministic. */
+ * token_copies is -1. Deterministic. */
 int sb_token_csr(const void* token_of_copy, int32_t token_is_i64, const int32_t* copy_row, int64_t num_copies,
                  int64_t num_tokens, int32_t* token_offsets, int32_t* token_copies, void* stream);
 

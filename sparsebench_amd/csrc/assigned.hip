@@ -8,12 +8,9 @@
 // no longer the k consecutive entries t*k .. t*k+k-1, so the reference sums
 // them with index_add_ (atomics, order not fixed). Here two steps replace it:
 //
-//   token_csr   one workgroup: token_offsets[T+1] and token_copies, the
-//               copies of each token in ascending copy order. Lists already
-//               ordered by token (top-k lists, token rounding's output) take
-//               a direct path: offsets from the run boundaries, copies = c.
-//               Other lists: histogram, scan, placement, then each token's
-//               few copies sorted, so the result does not depend on timing.
+//   token_csr   token_offsets[T+1] and token_copies, the copies of each token
+//               in ascending copy order. Each workgroup takes a run of tokens
+//               and reads the whole list, so no workgroup waits for another.
 //   combine     out[t] = bf16( sum over t's copies, in copy order, of
 //               fp32(y[copy_row[c]]) * fp32(weight[c]) ); 0 for no copies.
 //
@@ -29,112 +26,172 @@ namespace {
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kCsrThreads = 1024;
+constexpr int kCsrMaxTokens = 8192;  // of one workgroup
+constexpr int kCsrMaxCopies = 8192;  // of one workgroup, ranked in LDS
+constexpr int kCsrMaxList = 64;      // of one token, ranked in LDS
 
-// A copy is listed when routing placed it (copy_row >= 0; a bad expert or
-// token id, or a token >= valid_tokens, gives -1) and its token is in range.
+// Token of copy c, or -1 when it is not listed: routing did not place it
+// (copy_row < 0: a bad expert or token id, or a token >= valid_tokens) or its
+// token is out of range.
 template <typename Tok>
-__device__ __forceinline__ bool listed(const Tok* __restrict__ token, const int32_t* __restrict__ copy_row,
-                                       int64_t c, int32_t num_tokens) {
-  return copy_row[c] >= 0 && token[c] >= 0 && token[c] < static_cast<Tok>(num_tokens);
+__device__ __forceinline__ int32_t listed_token(const Tok* __restrict__ token, const int32_t* __restrict__ copy_row,
+                                                int64_t c, int64_t n, int32_t num_tokens) {
+  if (c >= n) return -1;
+  const int32_t row = copy_row[c];
+  const Tok t = token[c];
+  return row >= 0 && t >= 0 && t < static_cast<Tok>(num_tokens) ? static_cast<int32_t>(t) : -1;
 }
 
+// f(c, token) for every copy, lane-strided, kPer copies' loads in flight at
+// once (token -1: not listed).
+template <typename Tok, class F>
+__device__ __forceinline__ void for_each_copy(const Tok* __restrict__ token, const int32_t* __restrict__ copy_row,
+                                              int64_t n, int32_t num_tokens, F&& f) {
+  constexpr int kPer = 8;
+  for (int64_t base = threadIdx.x; base < n; base += kPer * kCsrThreads) {
+    int32_t t[kPer];
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) t[u] = listed_token(token, copy_row, base + u * kCsrThreads, n, num_tokens);
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) f(static_cast<int32_t>(base + u * kCsrThreads), t[u]);
+  }
+}
+
+// Sum of v over the workgroup, in every lane.
+__device__ __forceinline__ int32_t block_sum(int32_t v, int32_t* wave_sums) {
+  for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
+  if ((threadIdx.x & 63) == 0) wave_sums[threadIdx.x >> 6] = v;
+  __syncthreads();
+  int32_t sum = 0;
+  for (int w = 0; w < kCsrThreads / 64; ++w) sum += wave_sums[w];
+  __syncthreads();
+  return sum;
+}
+
+// Workgroup g takes tokens g * per .. +per. One pass over the whole list
+// counts its tokens' copies in LDS and the listed copies of the tokens
+// before them, which is where its copies start, so the workgroups need
+// nothing from each other; a second pass gathers its copies into their
+// tokens' slots, and each copy then moves to its rank within its token, so
+// the order does not depend on timing. (One workgroup with global atomics
+// took 41.7 us for 8192 copies of 4096 tokens, bound by their latency; this
+// takes 9.8: the list is read by every workgroup, 12 bytes a copy from L2.)
+// In a list already in token order (a top-k or a rounded list) the copies
+// are those slots themselves, and the second pass is left out.
+// Lists longer than kCsrMaxList, where the ranks cost more than they save,
+// and workgroups with more copies than the LDS holds take the slots in list
+// order instead, wave after wave.
 template <typename Tok>
 __global__ void __launch_bounds__(kCsrThreads)
     token_csr_kernel(const Tok* __restrict__ token, const int32_t* __restrict__ copy_row, int64_t n,
-                     int32_t num_tokens, int32_t* __restrict__ offsets, int32_t* __restrict__ copies) {
-  __shared__ int32_t total_listed;
-  const int tid = threadIdx.x;
-
-  // Direct path: every copy listed and tokens non-decreasing.
-  bool ordered = true;
-  for (int64_t c = tid; c < n; c += kCsrThreads) {
-    ordered = ordered && listed(token, copy_row, c, num_tokens) && (c == 0 || token[c] >= token[c - 1]);
-  }
-  if (__syncthreads_and(ordered)) {
-    // offsets[t] = first copy of a token >= t: copy c starts the tokens
-    // token[c-1]+1 .. token[c].
-    for (int64_t c = tid; c < n; c += kCsrThreads) {
-      const int64_t t = static_cast<int64_t>(token[c]);
-      const int64_t prev = c == 0 ? -1 : static_cast<int64_t>(token[c - 1]);
-      for (int64_t u = prev + 1; u <= t; ++u) offsets[u] = static_cast<int32_t>(c);
-      copies[c] = static_cast<int32_t>(c);
-    }
-    const int64_t last = n > 0 ? static_cast<int64_t>(token[n - 1]) : -1;
-    for (int64_t u = last + 1 + tid; u <= num_tokens; u += kCsrThreads) offsets[u] = static_cast<int32_t>(n);
-    return;
-  }
-
-  // General path. offsets[t+1] counts token t's copies ...
-  for (int64_t u = tid; u <= num_tokens; u += kCsrThreads) offsets[u] = 0;
-  __syncthreads();
-  for (int64_t c = tid; c < n; c += kCsrThreads)
-    if (listed(token, copy_row, c, num_tokens)) atomicAdd(&offsets[static_cast<int64_t>(token[c]) + 1], 1);
-  __syncthreads();
-  // ... an inclusive scan of it gives offsets[t+1] = end of token t.
+                     int32_t num_tokens, int32_t per, int32_t* __restrict__ offsets, int32_t* __restrict__ copies) {
+  __shared__ int32_t start[kCsrMaxTokens + 1];  // counts, then first slots (the workgroup's own numbering)
+  __shared__ int32_t next[kCsrMaxTokens];       // next free slot
+  __shared__ int32_t buf[kCsrMaxCopies];
+  __shared__ uint16_t buf_token[kCsrMaxCopies];
   __shared__ int32_t wave_sums[kCsrThreads / 64];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int32_t lo = static_cast<int32_t>(blockIdx.x) * per;
+  const int32_t mine = min(per, num_tokens - lo);
+  for (int i = tid; i < mine; i += kCsrThreads) start[i] = 0;
+  __syncthreads();
+
+  int32_t before = 0, all = 0;
+  bool ordered = true;
+  for_each_copy(token, copy_row, n, num_tokens, [&](int32_t c, int32_t t) {
+    all += t >= 0;
+    before += t >= 0 && t < lo;
+    if (t >= lo && t - lo < mine) atomicAdd(&start[t - lo], 1);
+    // The token before it, from the lane below; a wave's first lane reads it.
+    int32_t prev = __shfl_up(t, 1, 64);
+    if (lane == 0) prev = c > 0 && c < n ? static_cast<int32_t>(token[c - 1]) : 0;
+    ordered = ordered && (c >= n || (t >= 0 && t >= prev));
+  });
+  before = block_sum(before, wave_sums);  // synchronizes the workgroup
+  all = block_sum(all, wave_sums);
+
+  // start[i] = slots before token lo + i.
   int32_t carry = 0;
-  const int lane = tid & 63, wave = tid >> 6;
-  for (int64_t base = 1; base <= num_tokens; base += kCsrThreads) {
-    const int64_t u = base + tid;
-    int32_t v = u <= num_tokens ? offsets[u] : 0;
+  bool long_list = false;
+  for (int32_t base = 0; base < mine; base += kCsrThreads) {
+    const int32_t i = base + tid;
+    const int32_t own = i < mine ? start[i] : 0;
+    long_list = long_list || own > kCsrMaxList;
+    int32_t v = own;
     for (int d = 1; d < 64; d <<= 1) {
       const int32_t below = __shfl_up(v, d, 64);
       if (lane >= d) v += below;
     }
     if (lane == 63) wave_sums[wave] = v;
     __syncthreads();
-    int32_t before = carry;
-    for (int w = 0; w < wave; ++w) before += wave_sums[w];
-    int32_t chunk_total = 0;
-    for (int w = 0; w < kCsrThreads / 64; ++w) chunk_total += wave_sums[w];
-    if (u <= num_tokens) offsets[u] = v + before;
-    carry += chunk_total;
-    __syncthreads();
-  }
-  if (tid == 0) total_listed = carry;
-  __syncthreads();
-  // Placement: each copy takes a slot just below its token's end, which
-  // walks offsets[t+1] down to the start of token t ...
-  for (int64_t c = tid; c < n; c += kCsrThreads) {
-    if (!listed(token, copy_row, c, num_tokens)) continue;
-    const int32_t slot = atomicSub(&offsets[static_cast<int64_t>(token[c]) + 1], 1) - 1;
-    copies[slot] = static_cast<int32_t>(c);
-  }
-  __syncthreads();
-  // ... so offsets[t+1] now holds start(t): shift down by one, in passes
-  // of 8 entries per thread. A pass reads only entries above its own range,
-  // which earlier passes have not written.
-  constexpr int kPer = 8;
-  for (int64_t base = 0; base <= num_tokens; base += kPer * kCsrThreads) {
-    int32_t shifted[kPer];
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const int64_t u = base + i * kCsrThreads + tid;
-      shifted[i] = u < num_tokens ? offsets[u + 1] : total_listed;
+    int32_t sum = 0;
+    for (int w = 0; w < kCsrThreads / 64; ++w) {
+      if (w < wave) v += wave_sums[w];
+      sum += wave_sums[w];
     }
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < kPer; ++i) {
-      const int64_t u = base + i * kCsrThreads + tid;
-      if (u <= num_tokens) offsets[u] = shifted[i];
+    if (i < mine) {
+      start[i] = next[i] = carry + v - own;
+      offsets[lo + i] = before + carry + v - own;
     }
+    carry += sum;
     __syncthreads();
   }
-  // Each token's copies in ascending order (lists are a few entries long).
-  for (int64_t u = tid; u < num_tokens; u += kCsrThreads) {
-    const int32_t s = offsets[u], e = offsets[u + 1];
-    for (int32_t i = s + 1; i < e; ++i) {
-      const int32_t v = copies[i];
-      int32_t j = i - 1;
-      while (j >= s && copies[j] > v) {
-        copies[j + 1] = copies[j];
-        --j;
+  if (tid == 0) {
+    start[mine] = carry;
+    if (lo + mine == num_tokens) offsets[num_tokens] = all;
+  }
+  if (__syncthreads_and(ordered)) {  // every copy listed, in token order: a run of the list
+    for (int32_t i = tid; i < carry; i += kCsrThreads) copies[before + i] = before + i;
+  } else if (!__syncthreads_or(long_list || carry > kCsrMaxCopies)) {
+    for_each_copy(token, copy_row, n, num_tokens, [&](int32_t c, int32_t t) {
+      if (t >= lo && t - lo < mine) {
+        const int32_t slot = atomicAdd(&next[t - lo], 1);
+        buf[slot] = c;
+        buf_token[slot] = static_cast<uint16_t>(t - lo);
       }
-      copies[j + 1] = v;
+    });
+    __syncthreads();
+    for (int32_t i = tid; i < carry; i += kCsrThreads) {
+      const int32_t c = buf[i], s = start[buf_token[i]], e = start[buf_token[i] + 1];
+      int32_t rank = 0;
+      for (int32_t j = s; j < e; ++j) rank += buf[j] < c;
+      copies[before + s + rank] = c;
+    }
+  } else {
+    int bits = 0;
+    while ((1 << bits) < mine) ++bits;
+    for (int64_t base = 0; base < n; base += kCsrThreads) {
+      const int64_t c = base + tid;
+      const int32_t t = listed_token(token, copy_row, c, n, num_tokens) - lo;
+      const bool own = t >= 0 && t < mine;
+      uint64_t peers = __ballot(own);  // the wave's lanes with a copy of the same token
+      for (int b = 0; b < bits; ++b) {
+        const uint64_t ones = __ballot(own && ((t >> b) & 1));
+        peers &= ((t >> b) & 1) ? ones : ~ones;
+      }
+      const uint64_t lower = peers & ((uint64_t{1} << lane) - 1);
+      for (int w = 0; w < kCsrThreads / 64; ++w) {
+        if (w == wave && own) {
+          const int32_t slot = next[t];
+          copies[before + slot + __popcll(lower)] = static_cast<int32_t>(c);
+          if (lower == 0) next[t] = slot + __popcll(peers);
+        }
+        __syncthreads();
+      }
     }
   }
-  // Unused tail of the copy list.
-  for (int64_t c = static_cast<int64_t>(total_listed) + tid; c < n; c += kCsrThreads) copies[c] = -1;
+  // Unused tail of the copy list, shared by the workgroups.
+  for (int64_t c = static_cast<int64_t>(all) + static_cast<int64_t>(blockIdx.x) * kCsrThreads + tid; c < n;
+       c += static_cast<int64_t>(gridDim.x) * kCsrThreads)
+    copies[c] = -1;
+}
+
+// Tokens of one workgroup: 128 while that is at most one workgroup a CU,
+// then an equal share each, up to what its LDS holds, and fewer when they have
+// so many copies that half of the LDS would not hold them.
+int32_t csr_tokens_per_group(int64_t num_tokens, int64_t num_copies) {
+  const int64_t share = std::min<int64_t>(std::max<int64_t>(128, (num_tokens + 255) / 256), kCsrMaxTokens);
+  return static_cast<int32_t>(std::max<int64_t>(1, std::min(share, kCsrMaxCopies / 2 * num_tokens / num_copies)));
 }
 
 template <typename G>
@@ -213,14 +270,16 @@ extern "C" int sb_token_csr(const void* token_of_copy, int32_t token_is_i64, con
   if (!token_of_copy || !copy_row || !token_offsets || !token_copies)
     return fail(SB_ERR_INVALID, "token_csr: null buffer");
   const hipStream_t s = as_stream(stream);
+  const int32_t per = csr_tokens_per_group(num_tokens, num_copies);
+  const uint32_t groups = static_cast<uint32_t>((num_tokens + per - 1) / per);
   if (token_is_i64)
-    token_csr_kernel<int64_t><<<1, kCsrThreads, 0, s>>>(static_cast<const int64_t*>(token_of_copy), copy_row,
-                                                        num_copies, static_cast<int32_t>(num_tokens), token_offsets,
-                                                        token_copies);
+    token_csr_kernel<int64_t><<<groups, kCsrThreads, 0, s>>>(static_cast<const int64_t*>(token_of_copy), copy_row,
+                                                             num_copies, static_cast<int32_t>(num_tokens), per,
+                                                             token_offsets, token_copies);
   else
-    token_csr_kernel<int32_t><<<1, kCsrThreads, 0, s>>>(static_cast<const int32_t*>(token_of_copy), copy_row,
-                                                        num_copies, static_cast<int32_t>(num_tokens), token_offsets,
-                                                        token_copies);
+    token_csr_kernel<int32_t><<<groups, kCsrThreads, 0, s>>>(static_cast<const int32_t*>(token_of_copy), copy_row,
+                                                             num_copies, static_cast<int32_t>(num_tokens), per,
+                                                             token_offsets, token_copies);
   if (int rc = check_launch("token_csr")) return rc;
   return clear_ok();
 }
