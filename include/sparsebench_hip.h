@@ -234,6 +234,37 @@ int sb_token_rounding(const float* scores, int64_t num_tokens, int32_t num_exper
                       int32_t* row_token, int32_t* copy_row, int32_t* row_block_expert, int32_t* row_offsets,
                       int32_t* col_indices, int32_t* error, void* stream);
 
+/* ---- The whole layer in one call -------------------------------------- */
+
+/* Replace moe_forward, moe_forward_assigned (sparsebench/moe.py:25-91) and
+ * the rounded layer as one host call each: the stages above, enqueued on one
+ * stream with their intermediates (routing arrays, H, y) in `workspace`, a
+ * 256-byte aligned buffer of the size that the matching sizes call gives,
+ * free for other use once the stream has passed the call. x, w1 and w2 as in
+ * sb_sdd and sb_dsd (w2 [E, F, D]), out [T, D] bf16; the other arguments, the
+ * checks and the results are the stages' own. D % 256 == 0, F % 256 == 0, H
+ * (worst-case rows x F) and one expert's weights under 2 GiB, else
+ * SB_ERR_INVALID (the sizes call says so first): such shapes go through
+ * sb_sdd and sb_dsd.
+ * sb_layer_sizes: num_tokens = 0 for sb_layer (num_copies = T*k), T for
+ * sb_layer_assigned. */
+int sb_layer_sizes(int64_t num_tokens, int64_t num_copies, int64_t num_experts, int64_t d_model, int64_t ffn_dim,
+                   int64_t* workspace_bytes);
+int sb_layer_rounded_sizes(int64_t num_tokens, int32_t num_experts, int32_t k, int32_t tile, int64_t d_model,
+                           int64_t ffn_dim, int64_t* workspace_bytes);
+int sb_layer(const void* x, const void* expert_idx, int32_t idx_is_i64, const void* gates, int32_t gate_dtype,
+             const void* w1, const void* w2, void* out, void* workspace, int64_t workspace_bytes, int64_t num_tokens,
+             int32_t k, int32_t num_experts, int64_t d_model, int64_t ffn_dim, const int32_t* valid_tokens,
+             void* stream);
+int sb_layer_assigned(const void* x, const void* token_of_copy, int32_t token_is_i64, const void* expert_of_copy,
+                      int32_t expert_is_i64, const void* weights, int32_t weight_dtype, const void* w1,
+                      const void* w2, void* out, void* workspace, int64_t workspace_bytes, int64_t num_copies,
+                      int64_t num_tokens, int32_t num_experts, int64_t d_model, int64_t ffn_dim,
+                      const int32_t* valid_tokens, void* stream);
+int sb_layer_rounded(const void* x, const float* scores, const void* w1, const void* w2, void* out, void* workspace,
+                     int64_t workspace_bytes, int64_t num_tokens, int32_t num_experts, int32_t k, int32_t tile,
+                     int64_t d_model, int64_t ffn_dim, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

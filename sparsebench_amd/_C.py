@@ -15,6 +15,7 @@ kernel.
 from __future__ import annotations
 
 import ctypes
+import functools
 
 import torch
 
@@ -530,5 +531,122 @@ def token_rounding_cuda(scores: torch.Tensor, k: int, tile: int, ffn_dim: int, b
     check(lib().sb_token_rounding(
         scores.data_ptr(), num_tokens, num_experts, k, tile, block_size, ffn_dim, workspace.data_ptr(),
         *(t.data_ptr() for t in out.values()), stream_of(dev),
+    ))
+    return out
+
+
+# ---- the whole layer in one call (this build's C ABI): moe_forward and its
+# variants without stage marks ----
+
+_INDEX_DTYPES = {torch.int32: 0, torch.int64: 1}
+
+
+@functools.lru_cache(maxsize=256)
+def layer_bytes(num_tokens: int, num_copies: int, num_experts: int, d_model: int, ffn_dim: int) -> int | None:
+    """Workspace bytes of layer_cuda (num_tokens = 0) or layer_assigned_cuda; None for a
+    shape that the stages must take one by one (or refuse)."""
+    size = ctypes.c_int64()
+    if lib().sb_layer_sizes(num_tokens, num_copies, num_experts, d_model, ffn_dim, ctypes.byref(size)):
+        return None
+    return size.value
+
+
+@functools.lru_cache(maxsize=256)
+def layer_rounded_bytes(num_tokens: int, num_experts: int, k: int, tile: int, d_model: int, ffn_dim: int
+                        ) -> int | None:
+    """As layer_bytes, for layer_rounded_cuda."""
+    size = ctypes.c_int64()
+    if lib().sb_layer_rounded_sizes(num_tokens, num_experts, k, tile, d_model, ffn_dim, ctypes.byref(size)):
+        return None
+    return size.value
+
+
+def _layer_operands_ok(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor) -> bool:
+    """Whether the operands pass every check of the stages (which the caller falls back to, for their message)."""
+    dev = x.device
+    return (dev.type == "cuda" and w1.device == dev and w2.device == dev
+            and x.dtype is torch.bfloat16 and w1.dtype is torch.bfloat16 and w2.dtype is torch.bfloat16
+            and x.dim() == 2 and x.is_contiguous() and w1.is_contiguous() and w2.is_contiguous()
+            and not (x.data_ptr() | w1.data_ptr() | w2.data_ptr()) % 16)
+
+
+def _valid_tokens_ok(valid_tokens: torch.Tensor | None) -> bool:
+    return valid_tokens is None or (
+        valid_tokens.is_cuda and valid_tokens.dtype is torch.int32 and valid_tokens.numel() == 1)
+
+
+def layer_cuda(x: torch.Tensor, expert_idx: torch.Tensor, expert_weight: torch.Tensor, w1: torch.Tensor,
+               w2: torch.Tensor, valid_tokens: torch.Tensor | None) -> torch.Tensor | None:
+    """moe_forward's four stages as one call, or None when some operand or the
+    shape is not one that they all take as it is (then the stages say why).
+    Shapes are moe_forward's, checked there."""
+    num_experts, d_model, ffn_dim = w1.shape
+    num_tokens, k = x.shape[0], expert_idx.shape[-1]
+    idx_code, gate_code = _INDEX_DTYPES.get(expert_idx.dtype), _GATE_DTYPES.get(expert_weight.dtype)
+    if (idx_code is None or gate_code is None or expert_idx.dim() != 2 or num_tokens == 0 or k == 0
+            or not _layer_operands_ok(x, w1, w2) or not _valid_tokens_ok(valid_tokens)
+            or expert_idx.device != x.device or expert_weight.device != x.device
+            or not expert_idx.is_contiguous() or not expert_weight.is_contiguous()):
+        return None
+    size = layer_bytes(0, num_tokens * k, num_experts, d_model, ffn_dim)
+    if size is None:
+        return None
+    dev = x.device
+    workspace = torch.empty(size, dtype=torch.uint8, device=dev)
+    out = torch.empty(num_tokens, d_model, dtype=torch.bfloat16, device=dev)
+    check(lib().sb_layer(
+        x.data_ptr(), expert_idx.data_ptr(), idx_code, expert_weight.data_ptr(), gate_code, w1.data_ptr(),
+        w2.data_ptr(), out.data_ptr(), workspace.data_ptr(), size, num_tokens, k, num_experts, d_model, ffn_dim,
+        _ptr(valid_tokens), stream_of(dev),
+    ))
+    return out
+
+
+def layer_assigned_cuda(x: torch.Tensor, token_of_copy: torch.Tensor, expert_of_copy: torch.Tensor,
+                        weight_of_copy: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor,
+                        valid_tokens: torch.Tensor | None) -> torch.Tensor | None:
+    """moe_forward_assigned's stages as one call, or None as in layer_cuda. The
+    list's three tensors are 1-D, of one length, not empty."""
+    num_experts, d_model, ffn_dim = w1.shape
+    num_tokens, n = x.shape[0], expert_of_copy.numel()
+    token_code, expert_code = _INDEX_DTYPES.get(token_of_copy.dtype), _INDEX_DTYPES.get(expert_of_copy.dtype)
+    gate_code = _GATE_DTYPES.get(weight_of_copy.dtype)
+    dev = x.device
+    if (token_code is None or expert_code is None or gate_code is None or num_tokens == 0
+            or not _layer_operands_ok(x, w1, w2) or not _valid_tokens_ok(valid_tokens)
+            or token_of_copy.device != dev or expert_of_copy.device != dev or weight_of_copy.device != dev
+            or not token_of_copy.is_contiguous() or not expert_of_copy.is_contiguous()
+            or not weight_of_copy.is_contiguous()):
+        return None
+    size = layer_bytes(num_tokens, n, num_experts, d_model, ffn_dim)
+    if size is None:
+        return None
+    workspace = torch.empty(size, dtype=torch.uint8, device=dev)
+    out = torch.empty(num_tokens, d_model, dtype=torch.bfloat16, device=dev)
+    check(lib().sb_layer_assigned(
+        x.data_ptr(), token_of_copy.data_ptr(), token_code, expert_of_copy.data_ptr(), expert_code,
+        weight_of_copy.data_ptr(), gate_code, w1.data_ptr(), w2.data_ptr(), out.data_ptr(), workspace.data_ptr(), size,
+        n, num_tokens, num_experts, d_model, ffn_dim, _ptr(valid_tokens), stream_of(dev),
+    ))
+    return out
+
+
+def layer_rounded_cuda(x: torch.Tensor, scores: torch.Tensor, k: int, w1: torch.Tensor, w2: torch.Tensor,
+                       tile: int) -> torch.Tensor | None:
+    """moe_forward_rounded's stages as one call, or None as in layer_cuda."""
+    num_experts, d_model, ffn_dim = w1.shape
+    num_tokens = x.shape[0]
+    dev = x.device
+    if (not _layer_operands_ok(x, w1, w2) or scores.device != dev or scores.dtype is not torch.float32
+            or scores.dim() != 2 or not scores.is_contiguous() or num_tokens == 0):
+        return None
+    size = layer_rounded_bytes(num_tokens, num_experts, k, tile, d_model, ffn_dim)
+    if size is None:
+        return None
+    workspace = torch.empty(size, dtype=torch.uint8, device=dev)
+    out = torch.empty(num_tokens, d_model, dtype=torch.bfloat16, device=dev)
+    check(lib().sb_layer_rounded(
+        x.data_ptr(), scores.data_ptr(), w1.data_ptr(), w2.data_ptr(), out.data_ptr(), workspace.data_ptr(), size,
+        num_tokens, num_experts, k, tile, d_model, ffn_dim, stream_of(dev),
     ))
     return out

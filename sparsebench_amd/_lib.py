@@ -65,6 +65,20 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
         [_ptr, _i64, _i32, _i32, _i32, _i32, _i32, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr,
          _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _ptr],
     ),
+    "sb_layer_sizes": (_c_int, [_i64, _i64, _i64, _i64, _i64, ctypes.POINTER(_i64)]),
+    "sb_layer_rounded_sizes": (_c_int, [_i64, _i32, _i32, _i32, _i64, _i64, ctypes.POINTER(_i64)]),
+    "sb_layer": (
+        _c_int,
+        [_ptr, _ptr, _i32, _ptr, _i32, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i32, _i32, _i64, _i64, _ptr, _ptr],
+    ),
+    "sb_layer_assigned": (
+        _c_int,
+        [_ptr, _ptr, _i32, _ptr, _i32, _ptr, _i32, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i64, _i32, _i64, _i64, _ptr,
+         _ptr],
+    ),
+    "sb_layer_rounded": (
+        _c_int, [_ptr, _ptr, _ptr, _ptr, _ptr, _ptr, _i64, _i64, _i32, _i32, _i32, _i64, _i64, _ptr]
+    ),
 }
 
 SB_OK = 0

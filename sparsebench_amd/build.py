@@ -29,7 +29,7 @@ LIB_NAME = "libsparsebench_hip.so"
 PROBE_LIB_NAME = "libsparsebench_probe.so"
 ARCH = "gfx950"
 
-SOURCES = ["probe.hip", "routing.hip", "sdd.hip", "dsd.hip", "combine.hip", "assigned.hip", "router.hip", "experts.hip"]
+SOURCES = ["probe.hip", "routing.hip", "sdd.hip", "dsd.hip", "combine.hip", "assigned.hip", "router.hip", "experts.hip", "layer.hip"]
 PROBE_SOURCES = ["read_probe.hip", "schedule_shims.hip"]
 
 HIPCC_FLAGS = [
