@@ -20,6 +20,8 @@
 //               tokens_per_expert, or up to kScanChunks chunks from the
 //               counts, whose columns it then sums too
 //               (route_place_scan_kernel), in place of step 2.
+// Up to 1024 copies one launch does it all: every workgroup counts the one
+// chunk itself (route_one_chunk_kernel).
 // Place's two roles touch disjoint memory and depend only on steps 1-2.
 
 #include <mutex>
@@ -346,6 +348,73 @@ __global__ void __launch_bounds__(kChunk)
               row_block_expert, row_offsets, col_indices);
 }
 
+// Routing of one chunk in one launch: every workgroup counts the copies
+// itself (the per-wave counts of the placement, summed over the waves), scans
+// the padded sizes, and then workgroup 0 places and the others write the
+// layout, as in route_place_scan_kernel. Bound by latency, as its two-launch
+// form is (count 2.2 + place 4.7 us and the gap between them at 16 copies
+// over 64 experts; 4.6-5.1 us here). Beyond one chunk every workgroup would
+// repeat more counting than the launch costs.
+template <typename Idx, typename Tok>
+__global__ void __launch_bounds__(kChunk)
+    route_one_chunk_kernel(const Idx* __restrict__ idx, int64_t n, TokenSource<Tok> tokens, int32_t num_experts,
+                           int32_t num_bits, const int32_t* __restrict__ valid_tokens, int32_t block_size,
+                           int32_t ffn_blocks, int32_t max_row_blocks, int64_t max_rows,
+                           int32_t* __restrict__ tokens_per_expert, int32_t* __restrict__ padded_offsets,
+                           int32_t* __restrict__ error, int32_t* __restrict__ copy_row,
+                           int32_t* __restrict__ row_token, int32_t* __restrict__ row_block_expert,
+                           int32_t* __restrict__ row_offsets, int32_t* __restrict__ col_indices) {
+  __shared__ int32_t total[kMaxExperts];
+  __shared__ int32_t offs[kMaxExperts + 1];
+  __shared__ int32_t wave_counts[kWaves * kMaxExperts];
+  __shared__ int64_t wave_sums[kWaves];
+  const int tid = threadIdx.x, wave = tid >> 6;
+  const int waves = static_cast<int>((n + 63) / 64);  // waves with copies
+  bool bad = false;
+  int32_t token = -1;
+  const int32_t e = read_expert(idx, tid, n, tokens, num_experts, valid_tokens, &bad, &token);
+  for (int i = tid; i < waves * num_experts; i += kChunk) wave_counts[i] = 0;
+  const bool valid = e >= 0;
+  const uint64_t peers = same_expert_lanes(valid, e, num_bits);
+  const uint64_t lower = peers & lanes_below();
+  const bool any_bad = __syncthreads_or(bad);
+  if (valid && lower == 0) wave_counts[wave * num_experts + e] = __popcll(peers);  // one writer per (wave, e)
+  __syncthreads();
+  int32_t sum = 0;
+  if (tid < num_experts) {
+    for (int w = 0; w < waves; ++w) sum += wave_counts[w * num_experts + tid];
+    total[tid] = sum;
+  }
+  const int64_t padded = (static_cast<int64_t>(sum) + block_size - 1) / block_size * block_size;
+  const int64_t incl = block_inclusive_scan(padded, wave_sums);
+  if (tid < num_experts) offs[tid + 1] = static_cast<int32_t>(incl);
+  if (tid == 0) offs[0] = 0;
+  __syncthreads();
+  if (blockIdx.x == 0) {
+    if (tid < num_experts) {
+      tokens_per_expert[tid] = sum;
+      padded_offsets[tid + 1] = static_cast<int32_t>(incl);
+    }
+    if (tid == 0) {
+      padded_offsets[0] = 0;
+      error[0] = any_bad ? 1 : 0;
+    }
+    if (valid) {
+      int32_t before = 0;
+      for (int w = 0; w < wave; ++w) before += wave_counts[w * num_experts + e];
+      const int32_t row = offs[e] + before + __popcll(lower);
+      copy_row[tid] = row;
+      row_token[row] = token;
+    } else if (tid < n) {
+      copy_row[tid] = -1;
+    }
+    return;
+  }
+  const int64_t i = static_cast<int64_t>(blockIdx.x - 1) * kLayoutItemsPerGroup + tid;
+  layout_item(i, offs, total, num_experts, block_size, ffn_blocks, max_row_blocks, max_rows, row_token,
+              row_block_expert, row_offsets, col_indices);
+}
+
 int bits_for(int32_t num_experts) {
   int b = 0;
   while ((1 << b) < num_experts) ++b;
@@ -382,7 +451,8 @@ extern "C" int sb_routing_sizes(int64_t num_copies, int32_t num_experts, int32_t
 namespace sb {
 namespace {
 
-// Routing of n copies whose tokens come from `tokens`: count, then place with
+// Routing of n copies whose tokens come from `tokens`: one launch for one
+// chunk; else count, then place with
 // the column sums inside for at most kScanChunks chunks; count, columns and
 // place beyond.
 template <typename Idx, typename Tok>
@@ -398,6 +468,13 @@ int launch_routing(const Idx* idx, int64_t n, TokenSource<Tok> tokens, int32_t n
   const int64_t layout_items = std::max<int64_t>(max_row_blocks * ffn_blocks + 1, max_rows);
   const int32_t layout_groups = static_cast<int32_t>((layout_items + kLayoutItemsPerGroup - 1) / kLayoutItemsPerGroup);
 
+  if (num_chunks == 1) {
+    route_one_chunk_kernel<Idx, Tok><<<1 + layout_groups, kChunk, 0, stream>>>(
+        idx, n, tokens, num_experts, num_bits, valid_tokens, block_size, ffn_blocks,
+        static_cast<int32_t>(max_row_blocks), max_rows, tokens_per_expert, padded_offsets, error, copy_row, row_token,
+        row_block_expert, row_offsets, col_indices);
+    return check_launch("routing");
+  }
   route_count_kernel<Idx, Tok><<<num_chunks, kChunk, 0, stream>>>(idx, n, tokens, num_experts, num_bits,
                                                                   valid_tokens, workspace);
   if (int rc = check_launch("routing count")) return rc;
