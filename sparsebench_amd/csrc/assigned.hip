@@ -36,10 +36,11 @@ constexpr int kCsrMaxList = 64;      // of one token, ranked in LDS
 template <typename Tok>
 __device__ __forceinline__ int32_t listed_token(const Tok* __restrict__ token, const int32_t* __restrict__ copy_row,
                                                 int64_t c, int64_t n, int32_t num_tokens) {
-  if (c >= n) return -1;
-  const int32_t row = copy_row[c];
-  const Tok t = token[c];
-  return row >= 0 && t >= 0 && t < static_cast<Tok>(num_tokens) ? static_cast<int32_t>(t) : -1;
+  const int64_t at = min(c, n - 1);  // no branch: the caller's loads wait together
+  const int32_t row = copy_row[at];
+  const Tok t = token[at];
+  const bool listed = (c < n) & (row >= 0) & (t >= 0) & (t < static_cast<Tok>(num_tokens));
+  return listed ? static_cast<int32_t>(t) : -1;
 }
 
 // f(c, token) for every copy, lane-strided, kPer copies' loads in flight at

@@ -24,12 +24,13 @@
 //   3. select    one workgroup per expert: radix select (4 passes of 8 bits)
 //                of the target-th largest shifted score, then the keep
 //                bitmask, its per-word prefix counts and row_token.
-//   4. tokens    one wave per token: kept count and score total.
-//   5. scan      one workgroup: token_offsets (and the list length).
-//   6. emit      one wave per token: token / expert / weight / copy_row.
-//   7. layout    row_offsets, col_indices, row_block_expert, -1 rows.
+//   4. emit      one workgroup per 32 tokens (a word of every expert's
+//                bitmask): kept counts and score totals, token_offsets,
+//                token / expert / weight / copy_row; the other workgroups
+//                write row_offsets, col_indices, row_block_expert, -1 rows.
 
 #include "common.hpp"
+#include "expert_chunks.hpp"
 #include "layout.hpp"
 
 namespace sb {
@@ -39,7 +40,8 @@ constexpr int kTopkTokensPerGroup = 64;  // 4 waves x 16 tokens
 constexpr int kTopkThreads = 256;
 constexpr int kMaxPerLane = kMaxExperts / 64;
 constexpr int kSelectThreads = 1024;
-constexpr int kTokenWaves = 4;  // tokens kernel / emit kernel: waves per workgroup
+constexpr int kEmitThreads = 256;
+constexpr int kEmitWaves = kEmitThreads / 64;
 
 // Order-preserving map of a float to uint32 (larger float -> larger key).
 // -0 counts as +0 and every NaN as the largest value, as in a sort that
@@ -176,29 +178,57 @@ __global__ void __launch_bounds__(kTopkThreads)
       chunk_counts[static_cast<int64_t>(blockIdx.x) * num_experts + e] = hist[e];
 }
 
-// Top-k with one lane per token (a wave of 64 tokens per workgroup, the
-// same chunking as router_topk_kernel). The lane walks its token's row of
-// scores in expert order and keeps the KMAX best in registers, sorted by
-// (score desc, expert asc): each new (score, e) is bubbled in with
-// compare-and-swap steps, so an equal score behind an earlier expert stays
-// behind it. No lane talks to another, and the expert-major stores of the
-// shifted scores are 64 consecutive tokens per instruction. The outputs are
-// those of router_topk_kernel.
+// Top-k with one lane per token (64 tokens per workgroup, the same chunking
+// as router_topk_kernel). The workgroup's four waves read the scores a tile of
+// 64 tokens x up to kLaneTile experts at a time into LDS, whole rows of a
+// token side by side, and write the shifted scores from there; the first
+// wave's lanes walk their tokens' rows in the tile in expert order and keep
+// the KMAX best in registers, sorted by (score desc, expert asc): each new
+// (score, e) is bubbled in with compare-and-swap steps, so an equal score
+// behind an earlier expert stays behind it. No lane talks to another, and the
+// expert-major stores of the shifted scores are 64 consecutive tokens per
+// instruction. The outputs are those of router_topk_kernel. Bound by the
+// latency of its loads: with each lane reading its own row from memory,
+// twice, 13.6 us at T = 4096, E = 64, k = 2; this takes 8.3.
+constexpr int kLaneTile = 128;
+
 template <int KMAX>
-__global__ void __launch_bounds__(64)
+__global__ void __launch_bounds__(kTopkThreads)
     router_topk_lane_kernel(const float* __restrict__ scores, int64_t num_tokens, int32_t num_experts, int32_t k,
                             float* __restrict__ shifted, int32_t* __restrict__ chunk_counts,
                             int32_t* __restrict__ top_idx, float* __restrict__ top_weight) {
   __shared__ int32_t hist[kMaxExperts];
   __shared__ uint32_t picked_bits[64 * (kMaxExperts / 32)];  // lane-major: this lane's picks, one bit per expert
-  const int lane = threadIdx.x;
+  __shared__ float tile[64 * (kLaneTile + 1)];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int words = (num_experts + 31) / 32;
   if (chunk_counts != nullptr)
-    for (int e = lane; e < num_experts; e += 64) hist[e] = 0;
-  for (int w = 0; w < words; ++w) picked_bits[lane * words + w] = 0u;
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * 64 + lane;
-  const bool live = t < num_tokens;
-  const float* row = scores + (live ? t : 0) * num_experts;
+    for (int e = tid; e < num_experts; e += kTopkThreads) hist[e] = 0;
+  for (int w = tid; w < 64 * words; w += kTopkThreads) picked_bits[w] = 0u;
+  const int64_t t0 = static_cast<int64_t>(blockIdx.x) * 64;
+  const int64_t t = t0 + lane;
+  const int tokens = static_cast<int>(min(num_tokens - t0, int64_t{64}));
+  // Experts e0 .. e0+width of the workgroup's tokens; synchronizes around it.
+  auto load_tile = [&](int e0, int width) {
+    constexpr int kRows = 64 / (kTopkThreads / 64);  // tokens of a wave, all their loads in flight together
+    float v[kRows][kLaneTile / 64];
+#pragma unroll
+    for (int r = 0; r < kRows; ++r)
+#pragma unroll
+      for (int c = 0; c < kLaneTile / 64; ++c) {
+        const int tl = wave * kRows + r, e = 64 * c + lane;
+        // Past the tile: the last token or expert again (a load of its own
+        // branch for each would wait for the one before).
+        v[r][c] = scores[(t0 + min(tl, tokens - 1)) * num_experts + e0 + min(e, width - 1)];
+      }
+    __syncthreads();  // the tile before has been read
+#pragma unroll
+    for (int r = 0; r < kRows; ++r)
+#pragma unroll
+      for (int c = 0; c < kLaneTile / 64; ++c)
+        tile[(wave * kRows + r) * (kLaneTile + 1) + 64 * c + lane] = v[r][c];
+    __syncthreads();
+  };
 
   float bv[KMAX];
   int bi[KMAX];
@@ -209,38 +239,33 @@ __global__ void __launch_bounds__(64)
   }
   auto offer = [&](float v, int e) {
 #pragma unroll
-    for (int j = 0; j < KMAX; ++j) {
-      if (j < k && (bi[j] == 0x7fffffff || better(v, e, bv[j], bi[j]))) {
-        const float tv = bv[j];
-        const int ti = bi[j];
-        bv[j] = v;
-        bi[j] = e;
-        v = tv;
-        e = ti;
-      }
+    for (int j = 0; j < KMAX; ++j) {  // selects, not branches: the lanes disagree at every step
+      const bool in = (j < k) & ((bi[j] == 0x7fffffff) | (v > bv[j]) | ((v == bv[j]) & (e < bi[j])));
+      const float tv = in ? bv[j] : v;
+      const int ti = in ? bi[j] : e;
+      bv[j] = in ? v : bv[j];
+      bi[j] = in ? e : bi[j];
+      v = tv;
+      e = ti;
     }
   };
-  if (live) {
-    int e = 0;
-    if ((num_experts & 3) == 0 && (reinterpret_cast<uintptr_t>(scores) & 15) == 0) {
-      // 16 scores (four 16-byte loads) in flight at a time.
-      for (; e + 16 <= num_experts; e += 16) {
-        float4 q[4];
+  for (int e0 = 0; e0 < num_experts; e0 += kLaneTile) {
+    const int width = min(kLaneTile, num_experts - e0);
+    load_tile(e0, width);
+    if (wave == 0 && lane < tokens) {
+      constexpr int kBatch = 16;  // LDS reads in flight
+      int e = 0;
+      for (; e + kBatch <= width; e += kBatch) {
+        float v[kBatch];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) q[u] = *reinterpret_cast<const float4*>(row + e + 4 * u);
+        for (int u = 0; u < kBatch; ++u) v[u] = tile[lane * (kLaneTile + 1) + e + u];
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          offer(q[u].x, e + 4 * u);
-          offer(q[u].y, e + 4 * u + 1);
-          offer(q[u].z, e + 4 * u + 2);
-          offer(q[u].w, e + 4 * u + 3);
-        }
+        for (int u = 0; u < kBatch; ++u) offer(v[u], e0 + e + u);
       }
+      for (; e < width; ++e) offer(tile[lane * (kLaneTile + 1) + e], e0 + e);
     }
-    for (; e < num_experts; ++e) offer(row[e], e);
   }
-  __syncthreads();  // hist and picked_bits cleared
-  if (live) {
+  if (wave == 0 && lane < tokens) {
     float total = 0.0f;
 #pragma unroll
     for (int j = 0; j < KMAX; ++j) {
@@ -255,28 +280,29 @@ __global__ void __launch_bounds__(64)
 #pragma unroll
       for (int j = 0; j < KMAX; ++j)
         if (j < k) top_weight[t * k + j] = bv[j] / total;
-    if (shifted != nullptr) {
-      for (int e = 0; e < num_experts; ++e) {
-        const float v = row[e];
-        const bool pick = (picked_bits[lane * words + (e >> 5)] >> (e & 31)) & 1u;
-        shifted[static_cast<int64_t>(e) * num_tokens + t] = pick ? v : v - 1.0f;
-      }
+  }
+  __syncthreads();
+  if (shifted != nullptr) {
+    for (int e0 = 0; e0 < num_experts; e0 += kLaneTile) {
+      const int width = min(kLaneTile, num_experts - e0);
+      if (num_experts > kLaneTile) load_tile(e0, width);  // else the tile still holds all of them
+      if (lane < tokens)
+        for (int e = wave; e < width; e += kTopkThreads / 64) {
+          const float v = tile[lane * (kLaneTile + 1) + e];
+          const bool pick = (picked_bits[lane * words + ((e0 + e) >> 5)] >> ((e0 + e) & 31)) & 1u;
+          shifted[static_cast<int64_t>(e0 + e) * num_tokens + t] = pick ? v : v - 1.0f;
+        }
     }
   }
-  if (chunk_counts != nullptr) {
-    __syncthreads();
-    for (int e = lane; e < num_experts; e += 64)
+  if (chunk_counts != nullptr)
+    for (int e = tid; e < num_experts; e += kTopkThreads)
       chunk_counts[static_cast<int64_t>(blockIdx.x) * num_experts + e] = hist[e];
-  }
 }
 
 // Inclusive scan over the lanes of one 1024-lane workgroup.
 __device__ __forceinline__ int32_t block_scan_1024(int32_t v, int32_t* wave_sums, int32_t* total) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  for (int d = 1; d < 64; d <<= 1) {
-    const int32_t below = __shfl_up(v, d, 64);
-    if (lane >= d) v += below;
-  }
+  v = wave_inclusive_scan(v);
   if (lane == 63) wave_sums[wave] = v;
   __syncthreads();
   int32_t before = 0, all = 0;
@@ -344,6 +370,7 @@ __device__ __forceinline__ uint64_t lanes_below() {
 // would pile onto one or two addresses.
 __device__ __forceinline__ void wave_hist_add(int32_t* hist, uint32_t bin, bool active) {
   uint64_t peers = __ballot(active);
+  if (peers == 0) return;  // after the first pass or two, most waves
 #pragma unroll
   for (int b = 0; b < 8; ++b) {
     const bool bit = (bin >> b) & 1u;
@@ -361,11 +388,12 @@ __global__ void __launch_bounds__(kSelectThreads)
                          const int32_t* __restrict__ padded_offsets, uint32_t* __restrict__ keep_mask,
                          int32_t* __restrict__ keep_prefix, int32_t* __restrict__ row_token) {
   __shared__ uint32_t keys[kSelectLdsTokens];
-  __shared__ int32_t hist[256];
+  __shared__ int32_t hist[4][256];  // of each pass
   __shared__ int32_t wave_sums[16];
   __shared__ uint32_t s_prefix, s_prefix_mask;
+  __shared__ bool s_done;
   __shared__ int32_t s_remaining;
-  __shared__ int64_t s_cut;
+  __shared__ uint32_t counts[kSelectLdsTokens / 64];
   const int tid = threadIdx.x;
   const int e = blockIdx.x;
   const float* col = shifted + static_cast<int64_t>(e) * num_tokens;
@@ -383,7 +411,7 @@ __global__ void __launch_bounds__(kSelectThreads)
 #pragma unroll
       for (int u = 0; u < kPer; ++u) {
         const int64_t t = base + u * kSelectThreads + tid;
-        v[u] = t < num_tokens ? col[t] : 0.0f;
+        v[u] = col[min(t, num_tokens - 1)];
       }
 #pragma unroll
       for (int u = 0; u < kPer; ++u) {
@@ -395,10 +423,10 @@ __global__ void __launch_bounds__(kSelectThreads)
   }
   auto key_at = [&](int64_t t) -> uint32_t { return in_lds ? keys[t] : sort_key(col[t]); };
 
-  // Threshold key and the last tie kept: keep t iff key > thr, or
-  // key == thr and t <= cut.
+  // Keep t iff key > thr, or key == thr and fewer than `ties` tokens before it
+  // have that key.
   uint32_t thr = 0;
-  int64_t cut = -1;
+  int32_t ties = 0;
   bool keep_all = false, keep_none = false;
   if (tgt <= 0) {
     keep_none = true;
@@ -409,15 +437,18 @@ __global__ void __launch_bounds__(kSelectThreads)
       s_prefix = 0;
       s_prefix_mask = 0;
       s_remaining = tgt;
+      s_done = false;
     }
-    for (int shift = 24; shift >= 0; shift -= 8) {
-      for (int b = tid; b < 256; b += kSelectThreads) hist[b] = 0;
-      __syncthreads();
+    static_assert(kSelectThreads == 4 * 256, "one lane a bin of every pass");
+    hist[tid >> 8][tid & 255] = 0;
+    __syncthreads();
+    for (int pass = 0; pass < 4; ++pass) {
+      const int shift = 24 - 8 * pass;
       const uint32_t pre = s_prefix, pmask = s_prefix_mask;
       for (int64_t base = 0; base < num_tokens; base += kSelectThreads) {  // same trip count in every lane
         const int64_t t = base + tid;
         const uint32_t key = t < num_tokens ? key_at(t) : 0u;
-        wave_hist_add(hist, (key >> shift) & 255u, t < num_tokens && (key & pmask) == pre);
+        wave_hist_add(hist[pass], (key >> shift) & 255u, t < num_tokens && (key & pmask) == pre);
       }
       __syncthreads();
       if (tid < 64) {
@@ -427,14 +458,10 @@ __global__ void __launch_bounds__(kSelectThreads)
         int32_t c[4], own = 0;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          c[q] = hist[255 - 4 * tid - q];
+          c[q] = hist[pass][255 - 4 * tid - q];
           own += c[q];
         }
-        int32_t incl = own;  // keys in bins above and including this lane's four
-        for (int d = 1; d < 64; d <<= 1) {
-          const int32_t below = __shfl_up(incl, d, 64);
-          if (tid >= d) incl += below;
-        }
+        const int32_t incl = wave_inclusive_scan(own);  // keys in bins above and including this lane's four
         int32_t above = incl - own;  // keys in higher bins than this lane's
         // The lane whose four bins reach rem: the first with incl >= rem.
         const uint64_t reach = __ballot(incl >= rem);
@@ -442,9 +469,12 @@ __global__ void __launch_bounds__(kSelectThreads)
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
             if (above + c[q] >= rem) {
-              s_prefix = pre | (static_cast<uint32_t>(255 - 4 * tid - q) << shift);
+              const uint32_t found = pre | (static_cast<uint32_t>(255 - 4 * tid - q) << shift);
+              // All of the bin's keys are kept: keep every key above found - 1.
+              s_done = above + c[q] == rem && found != 0;
+              s_prefix = s_done ? found - 1 : found;
               s_prefix_mask = pmask | (255u << shift);
-              s_remaining = rem - above;
+              s_remaining = s_done ? 0 : rem - above;
               break;
             }
             above += c[q];
@@ -452,190 +482,187 @@ __global__ void __launch_bounds__(kSelectThreads)
         }
       }
       __syncthreads();
+      if (s_done) break;
     }
     thr = s_prefix;
-    const int32_t ties = s_remaining;  // keys == thr to keep, in token order
-    // The ties-th token with key == thr.
-    if (tid == 0) s_cut = num_tokens;
-    int32_t carry = 0;
-    for (int64_t base = 0; base < num_tokens; base += kSelectThreads) {
-      const int64_t t = base + tid;
-      const int32_t is_tie = (t < num_tokens && key_at(t) == thr) ? 1 : 0;
-      int32_t chunk_total;
-      const int32_t incl = block_scan_1024(is_tie, wave_sums, &chunk_total);
-      if (is_tie && carry + incl == ties) s_cut = t;
-      carry += chunk_total;
-      if (carry >= ties) break;  // uniform: every thread has the same carry
+    ties = s_remaining;  // keys == thr to keep, in token order
+  }
+
+  // Keep bitmask, 64 tokens a wave by ballot. The counts above and at the
+  // threshold of every 64 tokens of a round are scanned together (two halves
+  // of one word, each at most kSelectLdsTokens); a token's rank among the
+  // kept, its expert's row, follows from them.
+  constexpr int kRoundWaves = kSelectLdsTokens / 64;
+  static_assert(kRoundWaves <= kSelectThreads && kSelectLdsTokens < 65536, "one scan a round, two 16-bit counts");
+  const int lane = tid & 63, wave = tid >> 6;
+  const int32_t row0 = padded_offsets[e];
+  auto masks = [&](int64_t t, uint64_t* above, uint64_t* at) {
+    const bool in = t < num_tokens && !keep_none;
+    const uint32_t key = in && !keep_all ? key_at(t) : 0u;
+    *above = __ballot(in && (keep_all || key > thr));
+    *at = __ballot(in && !keep_all && key == thr);
+  };
+  int32_t above_before = 0, at_before = 0;  // of earlier rounds
+  for (int64_t base = 0; base < num_tokens; base += kSelectLdsTokens) {
+    const int waves = static_cast<int>(min((num_tokens - base + 63) / 64, static_cast<int64_t>(kRoundWaves)));
+    for (int w = wave; w < waves; w += kSelectThreads / 64) {
+      uint64_t above, at;
+      masks(base + 64 * w + lane, &above, &at);
+      if (lane == 0) counts[w] = (static_cast<uint32_t>(__popcll(above)) << 16) + __popcll(at);
     }
     __syncthreads();
-    cut = s_cut;
-  }
-
-  // Keep bitmask, one 32-token word per lane.
-  int32_t carry = 0;
-  for (int64_t base = 0; base < words; base += kSelectThreads) {
-    const int64_t w = base + tid;
-    uint32_t bits = 0;
-    if (w < words && !keep_none) {
-      for (int b = 0; b < 32; ++b) {
-        const int64_t t = w * 32 + b;
-        if (t >= num_tokens) break;
-        bool keep = keep_all;
-        if (!keep_all) {
-          const uint32_t key = key_at(t);
-          keep = key > thr || (key == thr && t <= cut);
-        }
-        if (keep) bits |= 1u << b;
+    int32_t total;
+    const int32_t mine = tid < waves ? static_cast<int32_t>(counts[tid]) : 0;
+    const int32_t incl = block_scan_1024(mine, wave_sums, &total);  // synchronizes the workgroup
+    if (tid < waves) counts[tid] = static_cast<uint32_t>(incl - mine);
+    __syncthreads();
+    for (int w = wave; w < waves; w += kSelectThreads / 64) {
+      const int64_t t = base + 64 * w + lane;
+      uint64_t above, at;
+      masks(t, &above, &at);
+      const int32_t tied = at_before + static_cast<int32_t>(counts[w] & 0xffffu);  // ties before these 64
+      const bool keep = ((above >> lane) & 1u) ||
+                        (((at >> lane) & 1u) && tied + __popcll(at & lanes_below()) < ties);
+      const uint64_t kept = __ballot(keep);
+      const int32_t first = above_before + static_cast<int32_t>(counts[w] >> 16) + min(tied, ties);
+      if (keep) row_token[row0 + first + __popcll(kept & lanes_below())] = static_cast<int32_t>(t);
+      const int64_t word = t / 32;
+      if ((lane & 31) == 0 && word < words) {
+        mask[word] = static_cast<uint32_t>(kept >> lane);
+        pref[word] = first + (lane == 0 ? 0 : __popc(static_cast<uint32_t>(kept)));
       }
     }
-    const int32_t cnt = __popc(bits);
-    int32_t chunk_total;
-    const int32_t incl = block_scan_1024(cnt, wave_sums, &chunk_total);
-    if (w < words) {
-      mask[w] = bits;
-      pref[w] = carry + incl - cnt;
-      // Kept tokens take the expert's rows in token order.
-      const int32_t row0 = padded_offsets[e] + carry + incl - cnt;
-      uint32_t rest = bits;
-      int32_t r = 0;
-      while (rest != 0) {
-        const int b = __builtin_ctz(rest);
-        rest &= rest - 1;
-        row_token[row0 + r] = static_cast<int32_t>(w * 32 + b);
-        ++r;
-      }
-    }
-    carry += chunk_total;
+    above_before += static_cast<int32_t>(static_cast<uint32_t>(total) >> 16);
+    at_before += total & 0xffff;
+    __syncthreads();
   }
 }
 
-// Kept experts of token t: bit e of word t/32 of expert e's mask.
-__device__ __forceinline__ bool kept(const uint32_t* __restrict__ keep_mask, int64_t words, int32_t e, int64_t t) {
-  return (keep_mask[static_cast<int64_t>(e) * words + (t >> 5)] >> (t & 31)) & 1u;
-}
-
-// One wave per token: number of kept experts and the sum of their scores,
-// added in ascending expert order.
-__global__ void __launch_bounds__(64 * kTokenWaves)
-    router_tokens_kernel(const float* __restrict__ scores, int64_t num_tokens, int32_t num_experts,
-                         const uint32_t* __restrict__ keep_mask, int32_t* __restrict__ kept_count,
-                         float* __restrict__ kept_total) {
-  const int lane = threadIdx.x & 63;
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * kTokenWaves + (threadIdx.x >> 6);
-  if (t >= num_tokens) return;
-  const int64_t words = (num_tokens + 31) / 32;
-  int32_t n = 0;
-  float total = 0.0f;
-  for (int e0 = 0; e0 < num_experts; e0 += 64) {
-    const int e = e0 + lane;
-    const bool keep = e < num_experts && kept(keep_mask, words, e, t);
-    const float s = keep ? scores[t * num_experts + e] : 0.0f;
-    uint64_t bal = __ballot(keep);
-    n += __popcll(bal);
-    while (bal != 0) {  // sequential, in expert order
-      const int l = __builtin_ctzll(bal);
-      bal &= bal - 1;
-      total += __shfl(s, l, 64);
-    }
-  }
-  if (lane == 0) {
-    kept_count[t] = n;
-    kept_total[t] = total;
-  }
-}
-
-// token_offsets = exclusive scan of kept_count; token_offsets[T] = N.
-// Each lane takes 16 consecutive tokens, so one workgroup scan covers 16K
-// tokens (one pass at the benchmark sizes).
-__global__ void __launch_bounds__(1024)
-    router_scan_kernel(const int32_t* __restrict__ kept_count, int64_t num_tokens, int32_t* __restrict__ token_offsets,
-                       int32_t* __restrict__ num_assignments) {
-  __shared__ int32_t wave_sums[16];
-  constexpr int kPer = 16;
-  int32_t carry = 0;
-  for (int64_t base = 0; base < num_tokens; base += 1024 * kPer) {
-    const int64_t t0 = base + static_cast<int64_t>(threadIdx.x) * kPer;
-    int32_t v[kPer];
-    int32_t own = 0;
-#pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      v[u] = t0 + u < num_tokens ? kept_count[t0 + u] : 0;
-      own += v[u];
-    }
-    int32_t chunk_total;
-    const int32_t incl = block_scan_1024(own, wave_sums, &chunk_total);
-    int32_t run = carry + incl - own;
-#pragma unroll
-    for (int u = 0; u < kPer; ++u) {
-      if (t0 + u < num_tokens) token_offsets[t0 + u] = run;
-      run += v[u];
-    }
-    carry += chunk_total;
-  }
-  if (threadIdx.x == 0) {
-    token_offsets[num_tokens] = carry;
-    num_assignments[0] = carry;
-  }
-}
-
-// One wave per token: its assignments, in expert order; then the unused
-// tail of copy_row (the capacity past N) is set to -1.
-__global__ void __launch_bounds__(64 * kTokenWaves)
+// Workgroup w < words: tokens 32 w .. 32 w + 31, one word of every expert's
+// keep bitmask. The copies of earlier tokens are the experts' prefix counts
+// at that word, so the workgroup finds its place in the list by itself; each
+// of its waves takes 8 tokens, a lane per expert: kept count, score total
+// (added in ascending expert order), then the token's entries in expert order.
+// The capacity past the list's end is filled with -1 / -1 / 0 / -1. The
+// workgroups past the words write the block-sparse layout. (Separate kernels
+// for counts, their scan, the list and the layout took 4.7 + 5.4 + 4.7 + 4.6
+// us at T = 4096, E = 64, each little more than its launch; this takes
+// 6.1.)
+template <int PER>
+__global__ void __launch_bounds__(kEmitThreads)
     router_emit_kernel(const float* __restrict__ scores, int64_t num_tokens, int32_t num_experts,
                        const uint32_t* __restrict__ keep_mask, const int32_t* __restrict__ keep_prefix,
-                       const float* __restrict__ kept_total, const int32_t* __restrict__ token_offsets,
-                       const int32_t* __restrict__ padded_offsets, int64_t capacity, int32_t* __restrict__ token_of_copy,
-                       int32_t* __restrict__ expert_of_copy, float* __restrict__ weight_of_copy,
-                       int32_t* __restrict__ copy_row) {
-  const int lane = threadIdx.x & 63;
-  const int64_t t = static_cast<int64_t>(blockIdx.x) * kTokenWaves + (threadIdx.x >> 6);
+                       const int32_t* __restrict__ tokens_per_expert, const int32_t* __restrict__ padded_offsets,
+                       int64_t capacity, int32_t block_size, int32_t ffn_blocks, int32_t max_row_blocks,
+                       int64_t max_rows, int32_t* __restrict__ token_offsets, int32_t* __restrict__ num_assignments,
+                       int32_t* __restrict__ token_of_copy, int32_t* __restrict__ expert_of_copy,
+                       float* __restrict__ weight_of_copy, int32_t* __restrict__ copy_row,
+                       int32_t* __restrict__ row_token, int32_t* __restrict__ row_block_expert,
+                       int32_t* __restrict__ row_offsets, int32_t* __restrict__ col_indices) {
+  constexpr int kPerWave = 32 / kEmitWaves;
+  __shared__ int32_t lds[2 * kMaxExperts + 1];
+  __shared__ int32_t sums[2][kEmitWaves];
+  __shared__ int32_t cnt[32];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int64_t words = (num_tokens + 31) / 32;
-  if (t < num_tokens) {
-    const float total = kept_total[t];
-    int32_t c = token_offsets[t];
-    for (int e0 = 0; e0 < num_experts; e0 += 64) {
-      const int e = e0 + lane;
-      const bool keep = e < num_experts && kept(keep_mask, words, e, t);
+  const int64_t word = blockIdx.x;
+  if (word >= words) {
+    int32_t* offs = lds;
+    int32_t* cnts = lds + kMaxExperts + 1;
+    for (int e = tid; e <= num_experts; e += kEmitThreads) offs[e] = padded_offsets[e];
+    for (int e = tid; e < num_experts; e += kEmitThreads) cnts[e] = tokens_per_expert[e];
+    __syncthreads();
+    layout_item((word - words) * kEmitThreads + tid, offs, cnts, num_experts, block_size, ffn_blocks, max_row_blocks,
+                max_rows, row_token, row_block_expert, row_offsets, col_indices);
+    return;
+  }
+  // The wave's tokens' scores, lane l the experts l, l + 64, ...: read whole,
+  // ahead of the bitmasks, so that their loads wait together.
+  float s[kPerWave][PER];
+#pragma unroll
+  for (int j = 0; j < kPerWave; ++j)
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int64_t t = min(word * 32 + wave * kPerWave + j, num_tokens - 1);
+      s[j][i] = scores[t * num_experts + min(64 * i + lane, num_experts - 1)];  // unused past the tokens and experts
+    }
+  uint32_t* mask = reinterpret_cast<uint32_t*>(lds);  // [E] this word of the experts' bitmasks
+  int32_t* row0 = lds + kMaxExperts;                  // [E] row of the expert's first kept token of the word
+  int32_t before = 0, all = 0;  // copies of earlier tokens, and of all
+  for (int e = tid; e < num_experts; e += kEmitThreads) {
+    const int64_t at = static_cast<int64_t>(e) * words + word;
+    const int32_t prefix = keep_prefix[at];
+    mask[e] = keep_mask[at];
+    row0[e] = padded_offsets[e] + prefix;
+    before += prefix;
+    all += tokens_per_expert[e];
+  }
+  before = wave_inclusive_scan_total(before);
+  all = wave_inclusive_scan_total(all);
+  if (lane == 0) {
+    sums[0][wave] = before;
+    sums[1][wave] = all;
+  }
+  __syncthreads();
+  before = all = 0;
+  for (int w = 0; w < kEmitWaves; ++w) {
+    before += sums[0][w];
+    all += sums[1][w];
+  }
+
+  float total[kPerWave];
+#pragma unroll
+  for (int j = 0; j < kPerWave; ++j) {
+    const int b = wave * kPerWave + j;
+    int32_t n = 0;
+    total[j] = 0.0f;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int e = 64 * i + lane;
+      uint64_t bal = __ballot(e < num_experts && ((mask[e] >> b) & 1u));  // never set past the tokens
+      n += __popcll(bal);
+      while (bal != 0) {  // sequential, in expert order
+        const int l = __builtin_ctzll(bal);
+        bal &= bal - 1;
+        total[j] += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(s[j][i]), l));
+      }
+    }
+    if (lane == 0) cnt[b] = n;
+  }
+  __syncthreads();
+  const int32_t own = lane < 32 ? cnt[lane] : 0;
+  const int32_t first = before + wave_inclusive_scan(own) - own;  // lane b < 32: where token b's entries start
+  if (wave == 0 && lane < 32 && word * 32 + lane < num_tokens) token_offsets[word * 32 + lane] = first;
+  if (word == words - 1 && tid == 0) {
+    token_offsets[num_tokens] = all;
+    num_assignments[0] = all;
+  }
+#pragma unroll
+  for (int j = 0; j < kPerWave; ++j) {
+    const int b = wave * kPerWave + j;
+    const int64_t t = word * 32 + b;
+    int32_t c = __builtin_amdgcn_readlane(first, b);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int e = 64 * i + lane;
+      const bool keep = e < num_experts && ((mask[e] >> b) & 1u);
       const uint64_t bal = __ballot(keep);
       if (keep) {
-        const int64_t slot = c + __popcll(bal & ((1ull << lane) - 1ull));
-        const uint32_t word = keep_mask[static_cast<int64_t>(e) * words + (t >> 5)];
-        const int32_t rank = keep_prefix[static_cast<int64_t>(e) * words + (t >> 5)] +
-                             __popc(word & ((1u << (t & 31)) - 1u));
+        const int64_t slot = c + __popcll(bal & lanes_below());
         token_of_copy[slot] = static_cast<int32_t>(t);
         expert_of_copy[slot] = e;
-        weight_of_copy[slot] = scores[t * num_experts + e] / total;
-        copy_row[slot] = padded_offsets[e] + rank;
+        weight_of_copy[slot] = s[j][i] / total[j];
+        copy_row[slot] = row0[e] + __popc(mask[e] & ((1u << b) - 1u));
       }
       c += __popcll(bal);
     }
   }
-  // Capacity tail.
-  const int64_t n = token_offsets[num_tokens];
-  const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
-  for (int64_t i = n + static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < capacity; i += stride) {
+  for (int64_t i = all + word * kEmitThreads + tid; i < capacity; i += words * kEmitThreads) {
     token_of_copy[i] = -1;
     expert_of_copy[i] = -1;
     weight_of_copy[i] = 0.0f;
     copy_row[i] = -1;
   }
-}
-
-constexpr int kLayoutItems = 1024;
-
-__global__ void __launch_bounds__(kLayoutItems)
-    router_layout_kernel(const int32_t* __restrict__ padded_offsets, const int32_t* __restrict__ tokens_per_expert,
-                         int32_t num_experts, int32_t block_size, int32_t ffn_blocks, int32_t max_row_blocks,
-                         int64_t max_rows, int32_t* __restrict__ row_token, int32_t* __restrict__ row_block_expert,
-                         int32_t* __restrict__ row_offsets, int32_t* __restrict__ col_indices) {
-  __shared__ int32_t offs[kMaxExperts + 1];
-  __shared__ int32_t cnts[kMaxExperts];
-  for (int e = threadIdx.x; e <= num_experts; e += kLayoutItems) offs[e] = padded_offsets[e];
-  for (int e = threadIdx.x; e < num_experts; e += kLayoutItems) cnts[e] = tokens_per_expert[e];
-  __syncthreads();
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * kLayoutItems + threadIdx.x;
-  layout_item(i, offs, cnts, num_experts, block_size, ffn_blocks, max_row_blocks, max_rows, row_token,
-              row_block_expert, row_offsets, col_indices);
 }
 
 struct RouterSizes {
@@ -662,7 +689,8 @@ int router_sizes(int64_t num_tokens, int32_t num_experts, int32_t k, int32_t til
   out->max_rows = rows;
   out->chunks = (num_tokens + kTopkTokensPerGroup - 1) / kTopkTokensPerGroup;
   out->words = (num_tokens + 31) / 32;
-  // chunk counts, target, shifted scores, keep mask, keep prefix, kept count, kept total
+  // chunk counts, shifted scores, keep mask, keep prefix; E + 2T words of the
+  // size that callers are told are spare
   out->workspace_elems = out->chunks * num_experts + num_experts + num_tokens * num_experts +
                          2 * out->words * num_experts + 2 * num_tokens;
   return SB_OK;
@@ -673,13 +701,15 @@ int launch_topk(const float* scores, int64_t num_tokens, int32_t num_experts, in
   const uint32_t groups = static_cast<uint32_t>((num_tokens + kTopkTokensPerGroup - 1) / kTopkTokensPerGroup);
   const int per = (num_experts + 63) / 64;
   // A lane per token unless its insertion work (E x the rounded-up k) is
-  // large; the test hook SB_HOOK_TOPK_KERNEL = 1 forces the wave form, 2
+  // large (4096 tokens, lane against wave form: E = 1000, k = 8 199 against
+  // 239 us; E = 512, k = 16 253 against 339; E = 1000, k = 16 491 against
+  // 472); the test hook SB_HOOK_TOPK_KERNEL = 1 forces the wave form, 2
   // the lane form.
   const int kmax = k <= 1 ? 1 : k <= 2 ? 2 : k <= 4 ? 4 : k <= 8 ? 8 : 16;
   const int forced = test_hook(SB_HOOK_TOPK_KERNEL);
-  if (forced == 2 || (forced != 1 && kmax * num_experts <= 2048)) {
+  if (forced == 2 || (forced != 1 && kmax * num_experts <= 8192)) {
 #define SB_TOPK_LANE(K) \
-  router_topk_lane_kernel<K><<<groups, 64, 0, s>>>(scores, num_tokens, num_experts, k, shifted, chunk_counts, top_idx, top_weight)
+  router_topk_lane_kernel<K><<<groups, kTopkThreads, 0, s>>>(scores, num_tokens, num_experts, k, shifted, chunk_counts, top_idx, top_weight)
     if (k <= 1) SB_TOPK_LANE(1);
     else if (k <= 2) SB_TOPK_LANE(2);
     else if (k <= 4) SB_TOPK_LANE(4);
@@ -748,12 +778,9 @@ extern "C" int sb_token_rounding(const float* scores, int64_t num_tokens, int32_
   const int32_t e = num_experts;
   // Workspace carve-up (int32 elements; the float arrays share the 4-byte slots).
   int32_t* chunk_counts = workspace;
-  int32_t* unused_target = chunk_counts + z.chunks * e;
-  float* shifted = reinterpret_cast<float*>(unused_target + e);
+  float* shifted = reinterpret_cast<float*>(chunk_counts + z.chunks * e);
   uint32_t* keep_mask = reinterpret_cast<uint32_t*>(shifted + t * e);
   int32_t* keep_prefix = reinterpret_cast<int32_t*>(keep_mask + z.words * e);
-  int32_t* kept_count = keep_prefix + z.words * e;
-  float* kept_total = reinterpret_cast<float*>(kept_count + t);
 
   if (int rc = launch_topk(scores, t, e, k, shifted, chunk_counts, nullptr, nullptr, s)) return rc;
   router_targets_kernel<<<1, 1024, 0, s>>>(chunk_counts, static_cast<int32_t>(z.chunks), e, t, tile, block_size,
@@ -762,23 +789,20 @@ extern "C" int sb_token_rounding(const float* scores, int64_t num_tokens, int32_
   router_select_kernel<<<e, kSelectThreads, 0, s>>>(shifted, t, tokens_per_expert, padded_offsets, keep_mask,
                                                     keep_prefix, row_token);
   if (int rc = check_launch("token rounding select")) return rc;
-  const uint32_t token_groups = static_cast<uint32_t>((t + kTokenWaves - 1) / kTokenWaves);
-  router_tokens_kernel<<<token_groups, 64 * kTokenWaves, 0, s>>>(scores, t, e, keep_mask, kept_count, kept_total);
-  if (int rc = check_launch("token rounding totals")) return rc;
-  router_scan_kernel<<<1, 1024, 0, s>>>(kept_count, t, token_offsets, num_assignments);
-  if (int rc = check_launch("token rounding scan")) return rc;
-  router_emit_kernel<<<token_groups, 64 * kTokenWaves, 0, s>>>(scores, t, e, keep_mask, keep_prefix, kept_total,
-                                                               token_offsets, padded_offsets, z.max_assignments,
-                                                               token_of_copy, expert_of_copy, weight_of_copy,
-                                                               copy_row);
-  if (int rc = check_launch("token rounding emit")) return rc;
   const int32_t ffn_blocks = ffn_dim / block_size;
   const int64_t layout_items = std::max<int64_t>(z.max_row_blocks * ffn_blocks + 1, z.max_rows);
-  const uint32_t layout_groups = static_cast<uint32_t>((layout_items + kLayoutItems - 1) / kLayoutItems);
-  router_layout_kernel<<<layout_groups, kLayoutItems, 0, s>>>(padded_offsets, tokens_per_expert, e, block_size,
-                                                              ffn_blocks, static_cast<int32_t>(z.max_row_blocks),
-                                                              z.max_rows, row_token, row_block_expert, row_offsets,
-                                                              col_indices);
-  if (int rc = check_launch("token rounding layout")) return rc;
+  const int64_t emit_groups = z.words + (layout_items + kEmitThreads - 1) / kEmitThreads;
+  auto emit = [&](auto per) {
+    router_emit_kernel<decltype(per)::value><<<static_cast<uint32_t>(emit_groups), kEmitThreads, 0, s>>>(
+        scores, t, e, keep_mask, keep_prefix, tokens_per_expert, padded_offsets, z.max_assignments, block_size,
+        ffn_blocks, static_cast<int32_t>(z.max_row_blocks), z.max_rows, token_offsets, num_assignments,
+        token_of_copy, expert_of_copy, weight_of_copy, copy_row, row_token, row_block_expert, row_offsets,
+        col_indices);
+  };
+  if (e <= 64) emit(std::integral_constant<int, 1>{});
+  else if (e <= 128) emit(std::integral_constant<int, 2>{});
+  else if (e <= 256) emit(std::integral_constant<int, 4>{});
+  else emit(std::integral_constant<int, kMaxPerLane>{});
+  if (int rc = check_launch("token rounding list")) return rc;
   return clear_ok();
 }

@@ -1,0 +1,43 @@
+"""Token rounding at the edges of its kernels: tokens around a word (32), a wave
+(64) and a round (32768) of the selection, experts around the widths of the
+top-k tile and of the list kernel, thresholds inside long runs of equal
+scores; bit for bit against the oracle, with the fused layout's list tail."""
+
+import numpy as np
+import pytest
+import torch
+
+from oracle.token_rounding_ref import token_rounding as token_rounding_ref
+
+pytestmark = pytest.mark.gpu
+
+
+def scores_of(t: int, e: int, levels: int) -> torch.Tensor:
+    """Scores in (0, 1), on `levels` values (ties everywhere), or continuous for 0."""
+    g = torch.Generator().manual_seed(t * 1000 + e)
+    s = torch.rand(t, e, generator=g).clamp_(1e-3, 0.999)
+    return s if levels == 0 else ((s * levels).floor() + 1) / (levels + 1)
+
+
+@pytest.mark.parametrize("levels", [0, 3])
+@pytest.mark.parametrize(("t", "e", "k", "tile"), [
+    (31, 5, 2, 4), (32, 64, 2, 4), (33, 65, 3, 4), (63, 128, 2, 8), (64, 129, 4, 8), (65, 255, 8, 8),
+    (1023, 256, 1, 16), (1025, 257, 2, 16), (130, 1024, 2, 4), (32768, 3, 1, 128), (32769, 3, 2, 128),
+    (65600, 2, 1, 128),
+])
+def test_list_matches_oracle(t: int, e: int, k: int, tile: int, levels: int) -> None:
+    from sparsebench_amd.routing import route_rounded
+
+    scores = scores_of(t, e, levels)
+    r = route_rounded(scores.cuda(), k, 256, 128, tile)
+    want = token_rounding_ref(scores.numpy(), k, tile)
+    n = want.token.size
+    assert int(r.num_assignments) == n and int(r.token_offsets[-1]) == n
+    for got, ref, fill in ((r.token_of_copy, want.token, -1), (r.expert_of_copy, want.expert, -1),
+                           (r.weight_of_copy, want.weight, 0)):
+        got = got.cpu().numpy()
+        assert np.array_equal(got[:n], ref) and np.all(got[n:] == fill)
+    assert np.array_equal(r.token_offsets.cpu().numpy()[:-1], np.searchsorted(want.token, np.arange(t)))
+    # copy_row and row_token name each other.
+    rows = r.topology.copy_row.cpu().numpy()
+    assert np.array_equal(r.topology.row_token.cpu().numpy()[rows[:n]], want.token) and np.all(rows[n:] == -1)
