@@ -41,6 +41,27 @@ inline int check_launch(const char* what) {
 // Only tests set them; the product path reads no environment.
 int32_t test_hook(int32_t hook);
 
+// CUs of the current device, read once per device; SB_OK or an error.
+int device_cus(int* cus);
+
+// The tiles' width for `units` tile rows of the per-row-block kernels: the
+// narrowest of 128, 256 and 512 that divides the columns and gives every tile
+// a CU of its own, else the widest. One CU takes in weights at a fixed rate
+// (53 GB/s from HBM), so a grid of few wide tiles is bound by one tile's
+// weights (DSD, D = 1024, F = 2048, E = 16, 19 row blocks: 48.6 us with 512
+// columns, 31.5 with 256, 25 with 128; D = 4096, F = 14336, 8 row blocks 309,
+// 230, 189), while with more tiles than CUs wider ones read less (D = 1024,
+// F = 4096, 127 row blocks: 136 us with 512 columns, 148 with 256, 180 with
+// 128).
+inline int fit_width(int64_t units, int64_t columns, int cus) {
+  int widest = 128;
+  for (int bn = 128; bn <= 512 && columns % bn == 0; bn *= 2) {
+    if (units * (columns / bn) <= cus) return bn;
+    widest = bn;
+  }
+  return widest;
+}
+
 // Row blocks per tile group (see tile_coords).
 constexpr int kTileGroup = 8;
 

@@ -41,27 +41,85 @@ int launch_dsd(const void* blocks, const void* w, const int32_t* row_offsets, co
   return check_launch("dsd");
 }
 
-// Tile shapes for a block size BM, from timing every shape tried on the
-// benchmark configurations (MI355X, samples interleaved across shapes):
-//   D % 512 == 0   128 x 512 tiles, BK 32 through a 4-stage ring, 4 waves of
-//                  128 x 128; with a deep reduction (K = F per expert >= 8192)
-//                  8 waves of 64 x 128
-//   D % 256 == 0   128 x 256 tiles, BK 64 x 3 stages, 8 waves
-//   otherwise      128 x 128 tiles, BK 64 x 3 stages, 4 waves
-// All with non-temporal W loads; the 256- and 512-wide ones issue the DMA of
-// a later step and the next sub-step's fragment reads among the MFMAs, and
-// the 512-wide ones load H two K steps at a time, as whole 128-byte rows
-// (APAIR; a row's K is a multiple of 64, since bs is 64 or 128), and read
-// the next step's first fragments among the current step's last MFMAs
-// (PIPE 5).
-template <int BM, class... Args>
-int dispatch_dsd(int64_t d_model, int64_t row_k, Args... args) {
-  if (d_model % 512 == 0) {
-    if (row_k >= 8192) return launch_dsd<DmaCfg<BM, 512, 32, 4, 2, 4, 0, 2, 5, 1, 1>>(args...);
-    return launch_dsd<DmaCfg<BM, 512, 32, 4, 1, 4, 0, 2, 5, 1, 1>>(args...);
+template <class Cfg>
+__global__ void __launch_bounds__(Cfg::kThreads)
+    dsd_pair_kernel(const uint16_t* __restrict__ blocks, const uint16_t* __restrict__ w,
+                    const int32_t* __restrict__ row_offsets, const int32_t* __restrict__ col_indices,
+                    uint16_t* __restrict__ out, int64_t nnz, int64_t w_rows, int32_t num_row_blocks, int32_t d_model,
+                    int32_t num_slices, int32_t zero_dead_rows) {
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[Cfg::kLdsAlloc];
+  dsd_pair_tile<Cfg, Cfg::BM / 2>(lds, static_cast<int>(blockIdx.x), blocks, w, row_offsets, col_indices, out, nnz,
+                                  w_rows, num_row_blocks, d_model, num_slices, zero_dead_rows, kTileGroup);
+}
+
+template <class Cfg>
+int launch_dsd_pairs(const void* blocks, const void* w, const int32_t* row_offsets, const int32_t* col_indices,
+                     void* out, int64_t nnz, int64_t w_rows, int64_t num_row_blocks, int64_t d_model,
+                     int32_t zero_dead_rows, hipStream_t stream) {
+  const int32_t num_slices = static_cast<int32_t>(d_model / Cfg::BN);
+  const int64_t groups = (num_row_blocks + 1) / 2 * 2 * num_slices;
+  dsd_pair_kernel<Cfg><<<static_cast<uint32_t>(groups), Cfg::kThreads, 0, stream>>>(
+      static_cast<const uint16_t*>(blocks), static_cast<const uint16_t*>(w), row_offsets, col_indices,
+      static_cast<uint16_t*>(out), nnz, w_rows, static_cast<int32_t>(num_row_blocks), static_cast<int32_t>(d_model),
+      num_slices, zero_dead_rows);
+  return check_launch("dsd");
+}
+
+// Tile shapes for BM rows, from timing every shape tried on the benchmark
+// configurations (MI355X, samples interleaved across shapes):
+//   512 wide  BK 32 through a 4-stage ring, 4 waves of BM x 128; with a deep
+//             reduction (K = F per expert >= 8192) 8 waves of BM/2 x 128
+//   256 wide  BK 64 x 3 stages, 8 waves
+//   128 wide  BK 64 x 3 stages, 4 waves
+// All with non-temporal W loads; they issue the DMA of a later step and the
+// next sub-step's fragment reads among the MFMAs, the 512-wide ones load H two
+// K steps at a time, as whole 128-byte rows (APAIR; a row's K is a multiple
+// of 64, since bs is 64 or 128), and those and the 128-wide ones read the next
+// step's first fragments among the current step's last MFMAs (PIPE 5).
+template <int BM>
+using DsdWide = DmaCfg<BM, 512, 32, 4, 1, 4, 0, 2, 5, 1, 1>;
+template <int BM>
+using DsdDeep = DmaCfg<BM, 512, 32, 4, 2, 4, 0, 2, 5, 1, 1>;
+template <int BM>
+using DsdMid = DmaCfg<BM, 256, 64, 3, 2, 4, 0, 2, 3>;
+template <int BM>
+using DsdNarrow = DmaCfg<BM, 128, 64, 3, 2, 2, 0, 2, 5>;
+
+template <class... Args>
+int dispatch_dsd_128(int64_t d_model, int64_t row_k, int64_t num_row_blocks, int cus, Args... args) {
+  switch (fit_width(num_row_blocks, d_model, cus)) {
+    case 512: return row_k >= 8192 ? launch_dsd<DsdDeep<128>>(args...) : launch_dsd<DsdWide<128>>(args...);
+    case 256: return launch_dsd<DsdMid<128>>(args...);
+    default: return launch_dsd<DsdNarrow<128>>(args...);
   }
-  if (d_model % 256 == 0) return launch_dsd<DmaCfg<BM, 256, 64, 3, 2, 4, 0, 2, 3>>(args...);
-  return launch_dsd<DmaCfg<BM, 128, 64, 3, 2, 2, 0, 2, 0>>(args...);
+}
+
+// Block size 64: row blocks one by one, or in pairs (dsd_pair_tile). A
+// routing layout of E experts has about (row blocks + E) / 2 tile rows in
+// pairs: the pairs, and row blocks alone, which cost a whole tile, at every
+// second expert's end. Pairs are taken when they let 512-wide tiles that leave
+// CUs idle become 256-wide ones (at least 4 row blocks an expert), or when
+// there are more tiles than CUs and at least 8 row blocks an expert. F = 2048,
+// E = 16, one by one against pairs: D = 1024, 79 row blocks 46 against 38 us;
+// D = 1024, 271 row blocks 127 against 107; but D = 4096, 79 row blocks 138
+// against 153, D = 512 (256 and 128 wide) 29 against 44, and with 3 row blocks
+// an expert (D = 1024, F = 4096, E = 64) 174 against 188.
+template <class... Args>
+int dispatch_dsd_64(int64_t d_model, int64_t row_k, int64_t w_rows, int64_t num_row_blocks, int cus, Args... args) {
+  const int64_t experts = row_k > 0 ? w_rows / row_k : num_row_blocks;
+  const int single = fit_width(num_row_blocks, d_model, cus);
+  const int paired = fit_width((num_row_blocks + experts) / 2, d_model, cus);
+  const bool narrower = single == 512 && paired == 256 && num_row_blocks >= 4 * experts;
+  const bool many = num_row_blocks * (d_model / single) > cus && num_row_blocks >= 8 * experts;
+  if (row_k < int64_t{64} * kMaxPairBlocks && paired >= 256 && (narrower || many)) {
+    if (paired == 256) return launch_dsd_pairs<DsdMid<128>>(args...);
+    return row_k >= 8192 ? launch_dsd_pairs<DsdDeep<128>>(args...) : launch_dsd_pairs<DsdWide<128>>(args...);
+  }
+  switch (single) {
+    case 512: return row_k >= 8192 ? launch_dsd<DsdDeep<64>>(args...) : launch_dsd<DsdWide<64>>(args...);
+    case 256: return launch_dsd<DsdMid<64>>(args...);
+    default: return launch_dsd<DsdNarrow<64>>(args...);
+  }
 }
 
 }  // namespace
@@ -92,9 +150,11 @@ extern "C" int sb_dsd(const void* blocks, const void* w, const int32_t* row_offs
   // num_row_blocks blocks per row), picks the deep-K tile.
   const int64_t row_k = nnz / num_row_blocks * block_size;
   const hipStream_t s = as_stream(stream);
+  int cus = 0;
+  if (const int rc = device_cus(&cus)) return rc;
   if (block_size == 128)
-    return dispatch_dsd<128>(d_model, row_k, blocks, w, row_offsets, col_indices, out, nnz, w_rows, num_row_blocks,
-                             d_model, zero_dead_rows, s);
-  return dispatch_dsd<64>(d_model, row_k, blocks, w, row_offsets, col_indices, out, nnz, w_rows, num_row_blocks,
-                          d_model, zero_dead_rows, s);
+    return dispatch_dsd_128(d_model, row_k, num_row_blocks, cus, blocks, w, row_offsets, col_indices, out, nnz, w_rows,
+                            num_row_blocks, d_model, zero_dead_rows, s);
+  return dispatch_dsd_64(d_model, row_k, w_rows, num_row_blocks, cus, blocks, w, row_offsets, col_indices, out, nnz,
+                         w_rows, num_row_blocks, d_model, zero_dead_rows, s);
 }

@@ -98,4 +98,134 @@ __device__ __forceinline__ void dsd_row_block_tile(uint8_t* __restrict__ lds, in
   });
 }
 
+// Two row blocks of BS rows over the same block columns, as one tile of
+// 2 BS rows: lane rows past BS read the second row block, `count` blocks on.
+// A row block alone: they read zeros (a_off past the buffer).
+template <class Cfg, int BS>
+struct DsdPairSrc {
+  static constexpr int kStepsPerBlock = BS / Cfg::BK;
+  static_assert(Cfg::BM == 2 * BS && (!Cfg::APAIR || kStepsPerBlock % 2 == 0), "pairs of row blocks");
+  const uint16_t* blocks;
+  const uint16_t* w;
+  const int32_t* col_indices;
+  int64_t w_rows;
+  int32_t d_model, begin, count;
+  uint32_t a_off[Cfg::kAInstr];
+  uint32_t b_off[Cfg::kBInstr];
+  __device__ __forceinline__ uint32_t a_voff(int q) const { return a_off[q]; }
+  __device__ __forceinline__ uint32_t b_voff(int q) const { return b_off[q]; }
+  __device__ __forceinline__ void a_src(int t, __amdgpu_buffer_rsrc_t* r, uint32_t* s) const {
+    *r = make_rsrc(blocks + static_cast<int64_t>(begin + t / kStepsPerBlock) * BS * BS,
+                   static_cast<uint32_t>(count + 1) * (BS * BS * 2u));
+    *s = static_cast<uint32_t>(t % kStepsPerBlock) * (Cfg::BK * 2);
+  }
+  __device__ __forceinline__ void b_src(int t, __amdgpu_buffer_rsrc_t* r, uint32_t* s) const {
+    const int64_t row0 = static_cast<int64_t>(col_indices[begin + t / kStepsPerBlock]) * BS;
+    const bool ok = row0 >= 0 && row0 + BS <= w_rows;
+    *r = make_rsrc(w + (ok ? row0 : 0) * d_model, ok ? static_cast<uint32_t>(BS) * d_model * 2u : 0u);
+    *s = static_cast<uint32_t>(t % kStepsPerBlock) * (Cfg::BK * 2u) * static_cast<uint32_t>(d_model);
+  }
+};
+
+constexpr int32_t kMaxPairBlocks = 1 << 16;  // of a row block, so that both row blocks' offsets fit 32 bits
+
+// Row blocks 2 pair and 2 pair + 1 of BS rows, from column n0 on, by two
+// workgroups (which = 0, 1): one tile of 2 BS rows by the first when both
+// have the same block columns, else a tile each, its second half of the rows
+// empty. Of 64-row blocks, most of a routing layout's are such pairs, and the
+// pair's tile reads its columns of w once for both. (One main loop for both
+// cases: beside a second one, for tiles of BS rows, the compiler loses the
+// ring's stages apart and waits for every load before each step's LDS reads.)
+template <class Cfg, int BS>
+__device__ __forceinline__ void dsd_pair_tile(uint8_t* __restrict__ lds, int bid, const uint16_t* __restrict__ blocks,
+                                              const uint16_t* __restrict__ w,
+                                              const int32_t* __restrict__ row_offsets,
+                                              const int32_t* __restrict__ col_indices, uint16_t* __restrict__ out,
+                                              int64_t nnz, int64_t w_rows, int32_t num_row_blocks, int32_t d_model,
+                                              int32_t num_slices, int32_t zero_dead_rows, int32_t group) {
+  using ML = DmaMainloop<Cfg>;
+  constexpr int BN = Cfg::BN;
+  // The first workgroups of all pairs' slices, then the second ones.
+  const int pairs = (num_row_blocks + 1) / 2;
+  const int which = uniform(bid / (pairs * num_slices));
+  const int live_rb = zero_dead_rows ? num_row_blocks : live_row_blocks(row_offsets, num_row_blocks);
+  const int live = (live_rb + 1) / 2;
+  // The second ones one by one over the XCDs: only those of row blocks alone
+  // have work, and several of them on one XCD would need a round of their own
+  // (D = 1024, 79 row blocks, by chance of the routing: 38 or 61 us).
+  const int id = bid - which * pairs * num_slices;
+  const int tile = which == 0 ? xcd_remap(id, live * num_slices) : id;
+  int pair, slice;
+  tile_coords(tile, live, num_slices, group, &pair, &slice);
+  if (pair >= pairs || which > 1) return;
+  const int n0 = slice * BN;
+  int rb = 2 * pair;
+
+  // Whether both row blocks have the same columns: all lanes' answer through
+  // the ring's LDS (__syncthreads_and would add its own to a full 160 KB).
+  bool same = rb + 1 < num_row_blocks;
+  if (same) {
+    const int32_t b0 = row_offsets[rb], b1 = row_offsets[rb + 1], b2 = row_offsets[rb + 2];
+    same = b0 >= 0 && b1 > b0 && b2 <= nnz && b2 - b1 == b1 - b0 && b1 - b0 < kMaxPairBlocks;
+    if (same)
+      for (int p = threadIdx.x; p < b1 - b0; p += Cfg::kThreads)
+        same = same && col_indices[b0 + p] == col_indices[b1 + p];
+  }
+  int32_t* agree = reinterpret_cast<int32_t*>(lds);
+  const bool wave_same = __ballot(!same) == 0;
+  if ((threadIdx.x & 63) == 0) agree[threadIdx.x >> 6] = wave_same ? 1 : 0;
+  __syncthreads();
+  int32_t waves_same = 0;
+  for (int v = 0; v < Cfg::kWaves; ++v) waves_same += agree[v];
+  const bool both = __builtin_amdgcn_readfirstlane(waves_same) == Cfg::kWaves;
+  __syncthreads();
+  if (both && which != 0) return;
+  if (!both) rb += which;
+  if (rb >= num_row_blocks) return;
+  int32_t begin = row_offsets[rb];
+  int32_t end = row_offsets[rb + 1];
+  if (begin < 0 || end > nnz || end < begin || end - begin >= kMaxPairBlocks) begin = end = 0;  // not a BSR row
+
+  uint16_t* out_tile = out + static_cast<int64_t>(rb) * BS * d_model + n0;
+  if (begin == end) {
+    if (!zero_dead_rows) return;
+    constexpr int kChunksPerRow = BN / 8;
+    for (int q = threadIdx.x; q < BS * kChunksPerRow; q += Cfg::kThreads) {
+      const int r = q / kChunksPerRow, c = q % kChunksPerRow;
+      *reinterpret_cast<u32x4_t*>(out_tile + static_cast<int64_t>(r) * d_model + c * 8) = u32x4_t{0u, 0u, 0u, 0u};
+    }
+    return;
+  }
+
+  DsdPairSrc<Cfg, BS> src;
+  src.blocks = blocks;
+  src.w = w + n0;
+  src.col_indices = col_indices;
+  src.w_rows = w_rows;
+  src.d_model = d_model;
+  src.begin = begin;
+  src.count = both ? end - begin : 0;
+  const ADmaPos<Cfg> ap;
+#pragma unroll
+  for (int q = 0; q < Cfg::kAInstr; ++q) {
+    const bool second = ap.row[q] >= BS;
+    const uint32_t at = (static_cast<uint32_t>(second ? end - begin : 0) * (BS * BS) + (ap.row[q] % BS) * BS +
+                         ap.chunk[q] * 8) * 2u;
+    src.a_off[q] = second && !both ? kOutOfRange : at;
+  }
+  const BDmaPos<Cfg> bp;
+#pragma unroll
+  for (int q = 0; q < Cfg::kBInstr; ++q)
+    src.b_off[q] = (static_cast<uint32_t>(bp.row[q]) * d_model + bp.col[q]) * 2u;
+
+  typename ML::Acc acc;
+  ML::run(lds, src, (end - begin) * DsdPairSrc<Cfg, BS>::kStepsPerBlock, acc);
+
+  const int rows = both ? 2 * BS : BS;
+  ML::stage_tile(lds, acc, [](float v) { return v; });
+  ML::for_each_staged_chunk(lds, [&](int r, int col, u32x4_t v) {
+    if (r < rows) *reinterpret_cast<u32x4_t*>(out_tile + static_cast<int64_t>(r) * d_model + col) = v;
+  });
+}
+
 }  // namespace sb

@@ -548,23 +548,6 @@ __global__ void __launch_bounds__(64 * WAVES)
 
 // --------------------------------------------------------------- launch ---
 
-// CUs of the current device, read once per device.
-int device_cus(int* cus_out) {
-  constexpr int kMaxDevices = 64;
-  static int cus[kMaxDevices] = {};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices)
-    return fail(SB_ERR_HIP, "dsd_experts: no current device");
-  if (cus[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
-      return fail(SB_ERR_HIP, "dsd_experts: cannot read the CU count");
-    cus[dev] = n;
-  }
-  *cus_out = cus[dev];
-  return SB_OK;
-}
-
 // Workgroups of dsd_layer_kernel: every row-block tile (the 512- or
 // 256-wide tile of sb_dsd's default shape), or every expert tile up to four
 // per CU if they can be more, and no more: workgroups past the chosen

@@ -20,6 +20,23 @@ int32_t test_hook(int32_t hook) {
   return hook >= 0 && hook < SB_NUM_TEST_HOOKS ? g_test_hooks[hook].load(std::memory_order_relaxed) : 0;
 }
 
+int device_cus(int* cus_out) {
+  constexpr int kMaxDevices = 64;
+  static std::atomic<int> cus[kMaxDevices];
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDevices)
+    return fail(SB_ERR_HIP, "no current device");
+  int known = cus[dev].load(std::memory_order_relaxed);
+  if (known == 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
+      return fail(SB_ERR_HIP, "cannot read the CU count");
+    cus[dev].store(known = n, std::memory_order_relaxed);
+  }
+  *cus_out = known;
+  return SB_OK;
+}
+
 int fail(int code, const char* fmt, ...) {
   char buf[512];
   va_list ap;
