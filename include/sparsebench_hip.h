@@ -134,6 +134,8 @@ int sb_dsd(const void* blocks, const void* w, const int32_t* row_offsets, const 
  * rows (the DSD's row-block tiles do not read them). It
  * calls sb_sdd itself when x or one expert's W1 is 2 GiB or more (the layer
  * kernels address them with 32-bit offsets).
+ * With so few live row blocks that tiles of 64, 128 or 256 columns (DSD: 64
+ * or 128) still have a CU each, the row blocks run as such narrow tiles.
  * The layout arrays are sb_routing's outputs (or those of
  * sb_routing_assigned / sb_token_rounding); max_row_blocks is its
  * worst-case row block count and num_copies the length of its copy_row.

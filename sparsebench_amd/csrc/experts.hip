@@ -23,6 +23,8 @@
 //        before it (RMAX 10): at the Mixtral-like shape every expert is then
 //        four chunks, 512 tiles in two rounds on 256 CUs, where a fifth,
 //        nearly empty chunk per expert made 592 tiles and a third round.
+// With few live row blocks both kernels run narrow tiles instead
+// (narrow_width, expert_chunks.hpp).
 // Rows of a chunk past its real rows are read as zeros (out-of-range DMA,
 // no memory read). SDD writes all 32 R rows of a chunk (padding rows as
 // GELU(0) = 0); DSD writes the real rows only. Padding rows past an
