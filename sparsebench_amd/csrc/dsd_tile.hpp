@@ -127,7 +127,9 @@ struct DsdPairSrc {
   }
 };
 
-constexpr int32_t kMaxPairBlocks = 1 << 16;  // of a row block, so that both row blocks' offsets fit 32 bits
+// Of a row block in a pair, so that both row blocks' offsets fit 32 bits. A row
+// block alone (count = 0: the buffer moves on with each block) has no limit.
+constexpr int32_t kMaxPairBlocks = 1 << 16;
 
 // Row blocks 2 pair and 2 pair + 1 of BS rows, from column n0 on, by two
 // workgroups (which = 0, 1): one tile of 2 BS rows by the first when both
@@ -184,7 +186,7 @@ __device__ __forceinline__ void dsd_pair_tile(uint8_t* __restrict__ lds, int bid
   if (rb >= num_row_blocks) return;
   int32_t begin = row_offsets[rb];
   int32_t end = row_offsets[rb + 1];
-  if (begin < 0 || end > nnz || end < begin || end - begin >= kMaxPairBlocks) begin = end = 0;  // not a BSR row
+  if (begin < 0 || end > nnz || end < begin) begin = end = 0;  // not a BSR row
 
   uint16_t* out_tile = out + static_cast<int64_t>(rb) * BS * d_model + n0;
   if (begin == end) {

@@ -78,6 +78,30 @@ def test_block_64_any_bsr(version: int) -> None:
         torch.testing.assert_close(out[r * 64:(r + 1) * 64].float().cpu(), want, **TOL)
 
 
+@pytest.mark.parametrize("version", [1, 4])
+def test_block_64_long_rows_among_short_ones(version: int) -> None:
+    # Row blocks of 65536 blocks (columns repeated), more than a pair takes, as the first and the second of theirs,
+    # in a layout that takes pairs. Small whole numbers: every sum is exact, up to the rounding of the result.
+    from types import SimpleNamespace
+
+    from sparsebench_amd.spmm import dsd
+
+    d, col_blocks, rows, long = 512, 8, 1024, {0, 3}
+    counts = torch.tensor([65536 if r in long else 8 for r in range(rows)])
+    offsets = torch.cat([torch.zeros(1, dtype=torch.int64), counts.cumsum(0)])
+    nnz = int(offsets[-1])
+    g = torch.Generator(device="cuda").manual_seed(4)
+    blocks = torch.randint(-1, 2, (nnz, 64, 64), generator=g, device="cuda", dtype=torch.int8).bfloat16()
+    w = torch.randint(-1, 2, (col_blocks * 64, d), generator=g, device="cuda", dtype=torch.int8).bfloat16()
+    topo = SimpleNamespace(block_size=64, row_offsets=offsets.int().cuda(),
+                           col_indices=(torch.arange(nnz, device="cuda") % col_blocks).int())
+    out = dsd(blocks, w, topo, version)
+    for r in (0, 1, 2, 3, 4, 5, rows - 1):
+        own = blocks[offsets[r]: offsets[r + 1]].view(-1, col_blocks, 64, 64).sum(0, dtype=torch.float32)
+        want = own.permute(1, 0, 2).reshape(64, -1).double() @ w.double()
+        assert torch.equal(out[r * 64: (r + 1) * 64], want.bfloat16()), r
+
+
 @pytest.mark.parametrize(("counts", "d", "f"), [
     ([100, 300], 256, 512), ([100, 300], 128, 8192), ([100, 300], 64, 16384), ([200, 5], 64, 33024), ([130], 64, 768),
 ])
