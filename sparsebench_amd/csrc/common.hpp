@@ -44,6 +44,18 @@ int32_t test_hook(int32_t hook);
 // CUs of the current device, read once per device; SB_OK or an error.
 int device_cus(int* cus);
 
+// sb_sdd_experts and sb_dsd_experts for a caller that knows how many rows its
+// routing places at least (min_rows, 0 when it does not): it only picks the
+// kernel instance. Results hold for any layout.
+int sdd_experts(const void* x, const void* w1, const int32_t* row_token, const int32_t* row_block_expert,
+                const int32_t* row_offsets, const int32_t* tokens_per_expert, const int32_t* padded_offsets, void* out,
+                int64_t num_tokens, int64_t d_model, int64_t ffn_dim, int64_t num_experts, int64_t max_row_blocks,
+                int64_t min_rows, int32_t apply_gelu, void* stream);
+int dsd_experts(const void* h, const void* w2, const int32_t* tokens_per_expert, const int32_t* padded_offsets,
+                const int32_t* row_block_expert, const int32_t* row_offsets, const int32_t* col_indices, void* out,
+                int64_t max_row_blocks, int64_t num_experts, int64_t num_copies, int64_t min_rows, int64_t ffn_dim,
+                int64_t d_model, void* stream);
+
 // The tiles' width for `units` tile rows of the per-row-block kernels: the
 // narrowest of 128, 256 and 512 that divides the columns and gives every tile
 // a CU of its own, else the widest. One CU takes in weights at a fixed rate

@@ -415,11 +415,27 @@ constexpr int kSddWidestNarrow = 256, kDsdWidestNarrow = 128;
 
 // The narrow tiles' width, or 0 for the wide tiles.
 __host__ __device__ __forceinline__ int narrow_width(int live_rb, int columns, int widest, int cus) {
-  if (live_rb <= 0 || live_rb > cus) return 0;
-#pragma unroll
-  for (int log_bn = 6; log_bn <= 8; ++log_bn)  // shifts: a division is a long sequence at every tile's start
-    if ((1 << log_bn) <= widest && static_cast<int64_t>(live_rb) * (columns >> log_bn) <= cus) return 1 << log_bn;
-  return 0;
+  // Every wide tile starts with this too, so its "no" comes first and costs a
+  // few scalar operations: no division, and 32-bit products (the first test
+  // bounds them).
+  const int log_widest = widest >= 256 ? 8 : 7;
+  if (live_rb <= 0 || live_rb > cus || (columns >> 8) > cus || live_rb * (columns >> log_widest) > cus) return 0;
+  if (live_rb * (columns >> 6) <= cus) return 64;
+  return live_rb * (columns >> 7) <= cus ? 128 : widest;
+}
+
+// Whether a stage's kernel is launched with the narrow tiles in it: unless
+// min_rows, the rows that the caller knows to be routed, already fill too many
+// row blocks for them. Beside them the wide tiles are slower (the width test
+// waits for padded_offsets before the counts are loaded, and takes scalar
+// registers): with against without, D = 2048, F = 2560, E = 8, 3962 Zipf
+// copies SDD 66.5 against 65.1 us, DSD 63.8 against 62.1; DSD of D = 1792,
+// F = 2048, E = 8, 10348 copies 104.2 against 103.0; SDD of D = 512, F = 7168,
+// E = 16, 14700 copies 199 against 194.
+inline bool may_be_narrow(int64_t min_rows, int64_t columns, int widest, int cus) {
+  const int64_t live_rb = (min_rows + kBS - 1) / kBS;  // at least
+  return live_rb <= 0 ||
+         (live_rb <= cus && narrow_width(static_cast<int>(live_rb), static_cast<int>(columns), widest, cus) > 0);
 }
 
 // Workgroup bid's narrow tile (rb >= live_rb: none), slice by slice within a

@@ -24,7 +24,7 @@
 //        four chunks, 512 tiles in two rounds on 256 CUs, where a fifth,
 //        nearly empty chunk per expert made 592 tiles and a third round.
 // With few live row blocks both kernels run narrow tiles instead
-// (narrow_width, expert_chunks.hpp).
+// (narrow_width, expert_chunks.hpp), in instances of their own (NARROW).
 // Rows of a chunk past its real rows are read as zeros (out-of-range DMA,
 // no memory read). SDD writes all 32 R rows of a chunk (padding rows as
 // GELU(0) = 0); DSD writes the real rows only. Padding rows past an
@@ -98,38 +98,35 @@ constexpr int max_int(int a, int b) { return a > b ? a : b; }
 
 // --------------------------------------------------------- narrow tiles ---
 
-// K steps of 64 through as deep a ring as 160 KB hold (up to 8 stages). The
-// computing waves are laid out to read each fragment as few times as can be;
-// the workgroup's other waves share the loads.
-template <int R, int BN, int WAVES>
+// K steps of 64 through as deep a ring (up to 8 stages) as the LDS of the
+// kernel's wide tiles holds: a ring that took more would cost the wide tiles
+// time (D = 1792, F = 3328, E = 8, DSD: 73.9 us with 128 KB a workgroup, 75.6
+// with 160, same code), and one CU's stream is as fast with 32 KB in flight
+// as with 128. The computing waves are laid out to read each fragment as few
+// times as can be; the workgroup's other waves share the loads.
+template <int R, int BN, int WAVES, int LDS>
 struct NarrowShape {
   static constexpr int WN = (BN == 256 && WAVES == 8 && R % 2 == 0) ? 4 : (BN / 32 < WAVES ? BN / 32 : WAVES);
   static constexpr int kRowWaves = WAVES / WN;
   static constexpr int WM = (R % 4 == 0 && kRowWaves >= 4) ? 4 : (R % 2 == 0 && kRowWaves >= 2) ? 2 : 1;
   static constexpr int XW = WAVES - WM * WN;
   static constexpr int kStage = (R * 4096 + 1024 * WAVES - 1) / (1024 * WAVES) * (1024 * WAVES) + BN * 128;
-  static constexpr int kFit = 160 * 1024 / kStage;
+  static constexpr int kFit = LDS / kStage;
   using Cfg = std::conditional_t<(R == 4 && BN == 256 && WAVES == 8), SddHalfTile,
                                  DmaCfg<32 * R, BN, 64, (kFit < 8 ? kFit : 8), WM, WN, 0, 2, 5, 1, 0, 0, XW>>;
   static_assert(Cfg::kThreads == 64 * WAVES, "the kernel's workgroup");
+  static_assert(Cfg::kLdsAlloc <= LDS, "the wide tiles' LDS");
 };
 
-template <int WAVES, int WIDEST, int R = 4>
-constexpr int narrow_lds_bytes() {
-  constexpr int own = max_int(max_int(NarrowShape<R, 64, WAVES>::Cfg::kLdsAlloc, NarrowShape<R, 128, WAVES>::Cfg::kLdsAlloc),
-                              NarrowShape<R, WIDEST, WAVES>::Cfg::kLdsAlloc);
-  if constexpr (R == 1) return own;
-  else return max_int(own, narrow_lds_bytes<WAVES, WIDEST, R - 1>());
-}
-
-// f(Tag<configuration>) for a narrow tile of `groups` row groups and `bn` columns.
-template <int WAVES, int WIDEST, class F>
+// f(Tag<configuration>) for a narrow tile of `groups` row groups and `bn`
+// columns, in a kernel of LDS bytes.
+template <int WAVES, int WIDEST, int LDS, class F>
 __device__ __forceinline__ void with_narrow(int groups, int bn, F&& f) {
   with_groups<4>(groups, [&](auto rc) {
     constexpr int R = decltype(rc)::value;
-    if (bn == 64) f(Tag<typename NarrowShape<R, 64, WAVES>::Cfg>{});
-    else if (bn == 128) f(Tag<typename NarrowShape<R, 128, WAVES>::Cfg>{});
-    else if constexpr (WIDEST >= 256) f(Tag<typename NarrowShape<R, 256, WAVES>::Cfg>{});
+    if (bn == 64) f(Tag<typename NarrowShape<R, 64, WAVES, LDS>::Cfg>{});
+    else if (bn == 128) f(Tag<typename NarrowShape<R, 128, WAVES, LDS>::Cfg>{});
+    else if constexpr (WIDEST >= 256) f(Tag<typename NarrowShape<R, 256, WAVES, LDS>::Cfg>{});
   });
 }
 
@@ -193,41 +190,41 @@ static_assert(SddChunkCfg<5>::kLdsAlloc <= 160 * 1024, "LDS");
 // Whether a narrow SDD tile of an expert of one row block may stop at its
 // last real 32-row group: when the DSD reads no further, as its 4-wave
 // row-block tiles and its narrow tiles do.
-__device__ __forceinline__ bool sdd_cuts_single(int live_rb, int ffn_dim, int d_model, int cus) {
-  return ffn_dim < kDsdDeepF || narrow_width(live_rb, d_model, kDsdWidestNarrow, cus) > 0;
+__device__ __forceinline__ bool sdd_cuts_single(int live_rb, int ffn_dim, int d_model, int cus, int dsd_narrow) {
+  return ffn_dim < kDsdDeepF || (dsd_narrow != 0 && narrow_width(live_rb, d_model, kDsdWidestNarrow, cus) > 0);
 }
 
-template <class CfgB>
+template <class CfgB, bool NARROW>
 __global__ void __launch_bounds__(64 * kSddWaves)
     sdd_layer_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w1,
                      const int32_t* __restrict__ row_token, const int32_t* __restrict__ row_block_expert,
                      const int32_t* __restrict__ row_offsets, const int32_t* __restrict__ tokens_per_expert,
                      const int32_t* __restrict__ padded_offsets, uint16_t* __restrict__ out, int32_t num_tokens,
                      int32_t d_model, int32_t ffn_dim, int32_t num_experts, int32_t max_row_blocks,
-                     int32_t apply_gelu, int32_t group, int32_t force, int32_t dsd_grid, int32_t cus_per_xcd,
-                     int32_t tail_slack) {
+                     int32_t apply_gelu, int32_t group, int32_t force, int32_t dsd_grid, int32_t dsd_narrow,
+                     int32_t cus_per_xcd, int32_t tail_slack) {
   static_assert(CfgB::kThreads == 64 * kSddWaves && CfgB::BM == kBS, "row-block tiles: 128 rows, same workgroup");
   using CfgH = SddHalfTile;
   static_assert(CfgH::kThreads == CfgB::kThreads && 2 * CfgH::BN == CfgB::BN, "half tiles: same workgroup");
-  __shared__ __attribute__((aligned(1024)))
-  uint8_t lds[max_int(max_int(max_int(chunk_lds_bytes<kSddBN, kSddWaves, kSddStages, kSddRmax>(),
+  constexpr int kLds = max_int(max_int(chunk_lds_bytes<kSddBN, kSddWaves, kSddStages, kSddRmax>(),
                                        chunk_lds_bytes<kSddBN, kSddWaves, 4, 4>()),
-                               max_int(CfgB::kLdsAlloc, CfgH::kLdsAlloc)),
-                       narrow_lds_bytes<kSddWaves, kSddWidestNarrow>())];
+                               max_int(CfgB::kLdsAlloc, CfgH::kLdsAlloc));
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kLds];
   // Workgroups past both tilings' tiles leave before the summary: every
   // chunk starts a row block of its own, so there are at most live row
   // blocks x slices tiles either way, numbered up to kNumXcd - 1 chunk rows
   // past them by the XCD deal, plus the split halves of a short last round.
+  int32_t first = 0;
+  if constexpr (!NARROW) first = expert_counts(tokens_per_expert, num_experts, 0);
   const int live_rb = __builtin_amdgcn_readfirstlane(padded_offsets[num_experts]) / kBS;
   const SddArgs a{x, w1, row_token, out, num_tokens, d_model, ffn_dim, apply_gelu};
   const int cus = cus_per_xcd * kNumXcd;
-  int32_t first;
   LayoutSummary sum;
   // The DSD's own choice (dsd_layer_kernel): its expert tiles when the
   // routing is balanced, F >= kDsdExpertMinF and its grid of dsd_grid
   // workgroups holds them all.
   auto expert_choice = [&] {
-    first = expert_counts(tokens_per_expert, num_experts, 0);
+    if constexpr (NARROW) first = expert_counts(tokens_per_expert, num_experts, 0);
     sum = summarize_layout<kSddRmax, 4, dsd_rmax<4>(), dsd_rmax<8>()>(tokens_per_expert, num_experts, first);
     const bool dsd_expert =
         force == 1 || (ffn_dim >= kDsdExpertMinF && expert_stage_runs(sum, num_experts, kGateDsd, force) &&
@@ -236,19 +233,21 @@ __global__ void __launch_bounds__(64 * kSddWaves)
                            dsd_grid);
     return expert_stage_runs(sum, num_experts, kGateSdd, force, ffn_dim / kSddBN, cus) && dsd_expert;
   };
-  const int bn = force == 0 ? narrow_width(live_rb, ffn_dim, kSddWidestNarrow, cus) : 0;
-  if (bn > 0) {
-    Chunk ch;
-    int slice;
-    if (!narrow_chunk(static_cast<int>(blockIdx.x), live_rb, ffn_dim / bn, row_block_expert, tokens_per_expert,
-                      padded_offsets, num_experts, max_row_blocks, sdd_cuts_single(live_rb, ffn_dim, d_model, cus),
-                      expert_choice, &ch, &slice))
+  if constexpr (NARROW) {
+    const int bn = force == 0 ? narrow_width(live_rb, ffn_dim, kSddWidestNarrow, cus) : 0;
+    if (bn > 0) {
+      Chunk ch;
+      int slice;
+      if (!narrow_chunk(static_cast<int>(blockIdx.x), live_rb, ffn_dim / bn, row_block_expert, tokens_per_expert,
+                        padded_offsets, num_experts, max_row_blocks,
+                        sdd_cuts_single(live_rb, ffn_dim, d_model, cus, dsd_narrow), expert_choice, &ch, &slice))
+        return;
+      with_narrow<kSddWaves, kSddWidestNarrow, kLds>(ch.groups, bn, [&](auto cfg) {
+        using Cfg = typename decltype(cfg)::type;
+        sdd_chunk_tile<Cfg>(lds, a, ch, slice * Cfg::BN);
+      });
       return;
-    with_narrow<kSddWaves, kSddWidestNarrow>(ch.groups, bn, [&](auto cfg) {
-      using Cfg = typename decltype(cfg)::type;
-      sdd_chunk_tile<Cfg>(lds, a, ch, slice * Cfg::BN);
-    });
-    return;
+    }
   }
   if (static_cast<int>(blockIdx.x) >= (live_rb + kNumXcd) * (ffn_dim / kSddBN) + tail_slack) return;
   if (!expert_choice()) {
@@ -347,42 +346,47 @@ __global__ void __launch_bounds__(64 * kSddWaves)
 // slices). Every padded row that a DSD tiling reads is written.
 using SddPairTile = DmaCfg<256, 256, 32, 4, 2, 4, 0, 2, 5, 1, 1>;
 
-template <class CfgP, class CfgS, class CfgSH>
+template <class CfgP, class CfgS, class CfgSH, bool NARROW>
 __global__ void __launch_bounds__(CfgP::kThreads)
     sdd_pair_kernel(const uint16_t* __restrict__ x, const uint16_t* __restrict__ w1,
                     const int32_t* __restrict__ row_token, const int32_t* __restrict__ row_block_expert,
                     const int32_t* __restrict__ tokens_per_expert, const int32_t* __restrict__ padded_offsets,
                     uint16_t* __restrict__ out, int32_t num_tokens, int32_t d_model, int32_t ffn_dim,
                     int32_t num_experts, int32_t max_row_blocks, int32_t apply_gelu, int32_t force,
-                    int32_t cus_per_xcd) {
+                    int32_t dsd_narrow, int32_t cus_per_xcd) {
   static_assert(CfgP::kThreads == CfgS::kThreads && CfgP::BN == CfgS::BN, "one workgroup and slice width");
   static_assert(CfgSH::kThreads == CfgS::kThreads && 2 * CfgSH::BN == CfgS::BN && CfgSH::BK == CfgS::BK,
                 "a single's column halves: same workgroup and K steps");
   static_assert(CfgP::BM == 2 * kBS && CfgS::BM == kBS && CfgSH::BM == kBS, "pairs and singles of row blocks");
-  __shared__ __attribute__((aligned(1024)))
-  uint8_t lds[max_int(max_int(CfgP::kLdsAlloc, narrow_lds_bytes<kSddWaves, kSddWidestNarrow>()),
-                      max_int(CfgS::kLdsAlloc, CfgSH::kLdsAlloc))];
-  // Workgroup bid is XCD bid % 8's tile bid / 8 (units x slices, unit-major,
-  // a short last round of singles as column halves; pair_tile_for).
+  constexpr int kLds = NARROW ? 160 * 1024 : max_int(CfgP::kLdsAlloc, max_int(CfgS::kLdsAlloc, CfgSH::kLdsAlloc));
+  static_assert(CfgP::kLdsAlloc <= kLds && CfgS::kLdsAlloc <= kLds && CfgSH::kLdsAlloc <= kLds, "LDS");
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kLds];
+  int32_t first = 0;
+  if constexpr (!NARROW) first = expert_counts(tokens_per_expert, num_experts, 0);
   const int live_rb = __builtin_amdgcn_readfirstlane(padded_offsets[num_experts]) / kBS;
   const int slices = ffn_dim / CfgP::BN;
   const SddArgs a{x, w1, row_token, out, num_tokens, d_model, ffn_dim, apply_gelu};
-  const int bn = force == 0 ? narrow_width(live_rb, ffn_dim, kSddWidestNarrow, cus_per_xcd * kNumXcd) : 0;
-  if (bn > 0) {
-    Chunk nch;
-    int nslice;
-    if (!narrow_chunk(static_cast<int>(blockIdx.x), live_rb, ffn_dim / bn, row_block_expert, tokens_per_expert,
-                      padded_offsets, num_experts, max_row_blocks,
-                      sdd_cuts_single(live_rb, ffn_dim, d_model, cus_per_xcd * kNumXcd), [] { return false; }, &nch,
-                      &nslice))
+  if constexpr (NARROW) {
+    const int cus = cus_per_xcd * kNumXcd;
+    const int bn = force == 0 ? narrow_width(live_rb, ffn_dim, kSddWidestNarrow, cus) : 0;
+    if (bn > 0) {
+      Chunk nch;
+      int nslice;
+      if (!narrow_chunk(static_cast<int>(blockIdx.x), live_rb, ffn_dim / bn, row_block_expert, tokens_per_expert,
+                        padded_offsets, num_experts, max_row_blocks,
+                        sdd_cuts_single(live_rb, ffn_dim, d_model, cus, dsd_narrow), [] { return false; }, &nch,
+                        &nslice))
+        return;
+      with_narrow<kSddWaves, kSddWidestNarrow, kLds>(nch.groups, bn, [&](auto cfg) {
+        using Cfg = typename decltype(cfg)::type;
+        sdd_chunk_tile<Cfg>(lds, a, nch, nslice * Cfg::BN);
+      });
       return;
-    with_narrow<kSddWaves, kSddWidestNarrow>(nch.groups, bn, [&](auto cfg) {
-      using Cfg = typename decltype(cfg)::type;
-      sdd_chunk_tile<Cfg>(lds, a, nch, nslice * Cfg::BN);
-    });
-    return;
+    }
+    first = expert_counts(tokens_per_expert, num_experts, 0);
   }
-  const int32_t first = expert_counts(tokens_per_expert, num_experts, 0);
+  // Workgroup bid is XCD bid % 8's tile bid / 8 (units x slices, unit-major,
+  // a short last round of singles as column halves; pair_tile_for).
   if (static_cast<int>(blockIdx.x) / kNumXcd >= pair_units_per_xcd(live_rb) * slices + cus_per_xcd / 2) return;
   const PairCounts pc = pair_counts(tokens_per_expert, num_experts, first);
   bool single;
@@ -429,7 +433,7 @@ __global__ void __launch_bounds__(CfgP::kThreads)
 // expert chunks (one H buffer, K steps through the row block's own F/128
 // blocks, as the routing layout stores them).
 
-template <class CfgB, int WAVES>
+template <class CfgB, int WAVES, bool NARROW>
 __global__ void __launch_bounds__(64 * WAVES)
     dsd_layer_kernel(const uint16_t* __restrict__ h, const uint16_t* __restrict__ w2,
                      const int32_t* __restrict__ tokens_per_expert, const int32_t* __restrict__ padded_offsets,
@@ -439,34 +443,40 @@ __global__ void __launch_bounds__(64 * WAVES)
   static_assert(CfgB::kThreads == 64 * WAVES && CfgB::BM == kBS, "row-block tiles: 128 rows, same workgroup");
   using CfgH = DsdCfg<4, CfgB::BN / 2, WAVES, kDsdStages>;
   constexpr int kRmax = dsd_rmax<WAVES>();
-  __shared__ __attribute__((aligned(1024)))
-  uint8_t lds[max_int(max_int(chunk_lds_bytes<kDsdBN, WAVES, kDsdStages, kRmax>(), narrow_lds_bytes<WAVES, kDsdWidestNarrow>()),
-                      max_int(CfgB::kLdsAlloc, CfgH::kLdsAlloc))];
+  constexpr int kLds =
+      max_int(chunk_lds_bytes<kDsdBN, WAVES, kDsdStages, kRmax>(), max_int(CfgB::kLdsAlloc, CfgH::kLdsAlloc));
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kLds];
+  int32_t first = 0;
+  if constexpr (!NARROW) first = expert_counts(tokens_per_expert, num_experts, 0);
   const int live_rb = __builtin_amdgcn_readfirstlane(padded_offsets[num_experts]) / kBS;
   const DsdArgs a{h, w2, out, h_bytes, ffn_dim, d_model};
-  int32_t first;
   LayoutSummary sum;
   // Expert tiles for balanced routing over a reduction of at least
   // kDsdExpertMinF. The grid may hold fewer workgroups than expert tiles
   // (see the launch): then the row blocks take the stage.
   auto expert_choice = [&] {
-    first = expert_counts(tokens_per_expert, num_experts, 0);
+    if constexpr (NARROW) first = expert_counts(tokens_per_expert, num_experts, 0);
     sum = summarize_layout<kRmax, 4>(tokens_per_expert, num_experts, first);
     const bool fits = static_cast<int64_t>(sum.chunks_a) * (d_model / kDsdBN) <= static_cast<int64_t>(tile_grid);
-    return force == 1 || (ffn_dim >= kDsdExpertMinF && expert_stage_runs(sum, num_experts, kGateDsd, force) && fits);
+    // (force tested last: tested first it splits the flow here, and the compiler
+    // then recomputes A addresses in the 128 x 512 tile's main loop.)
+    const bool chosen = ffn_dim >= kDsdExpertMinF && expert_stage_runs(sum, num_experts, kGateDsd, force) && fits;
+    return chosen || force == 1;
   };
-  const int bn = force == 0 ? narrow_width(live_rb, d_model, kDsdWidestNarrow, cus_per_xcd * kNumXcd) : 0;
-  if (bn > 0) {
-    Chunk ch;
-    int slice;
-    if (!narrow_chunk(static_cast<int>(blockIdx.x), live_rb, d_model / bn, row_block_expert, tokens_per_expert,
-                      padded_offsets, num_experts, max_row_blocks, true, expert_choice, &ch, &slice))
+  if constexpr (NARROW) {
+    const int bn = force == 0 ? narrow_width(live_rb, d_model, kDsdWidestNarrow, cus_per_xcd * kNumXcd) : 0;
+    if (bn > 0) {
+      Chunk ch;
+      int slice;
+      if (!narrow_chunk(static_cast<int>(blockIdx.x), live_rb, d_model / bn, row_block_expert, tokens_per_expert,
+                        padded_offsets, num_experts, max_row_blocks, true, expert_choice, &ch, &slice))
+        return;
+      with_narrow<WAVES, kDsdWidestNarrow, kLds>(ch.groups, bn, [&](auto cfg) {
+        using Cfg = typename decltype(cfg)::type;
+        dsd_chunk_tile<Cfg>(lds, a, ch, slice * Cfg::BN);
+      });
       return;
-    with_narrow<WAVES, kDsdWidestNarrow>(ch.groups, bn, [&](auto cfg) {
-      using Cfg = typename decltype(cfg)::type;
-      dsd_chunk_tile<Cfg>(lds, a, ch, slice * Cfg::BN);
-    });
-    return;
+    }
   }
   // As in the SDD: at most live row blocks x D/256 tiles either way, plus
   // the split halves of a short last round.
@@ -580,7 +590,7 @@ template <class CfgB>
 int launch_sdd_layer(const void* x, const void* w1, const int32_t* row_token, const int32_t* row_block_expert,
                      const int32_t* row_offsets, const int32_t* tokens_per_expert, const int32_t* padded_offsets,
                      void* out, int64_t num_tokens, int64_t d_model, int64_t ffn_dim, int64_t num_experts,
-                     int64_t max_row_blocks, int32_t apply_gelu, int32_t force, hipStream_t stream) {
+                     int64_t max_row_blocks, int64_t min_rows, int32_t apply_gelu, int32_t force, hipStream_t stream) {
   // Both tilings have at most max_row_blocks x F/512 tiles (every chunk
   // starts a row block of its own).
   static_assert(CfgB::BN == kSddBN, "one grid for both tilings");
@@ -595,33 +605,38 @@ int launch_sdd_layer(const void* x, const void* w1, const int32_t* row_token, co
   int cus = 0;
   if (const int rc = device_cus(&cus)) return rc;
   const int64_t slack = split_tail_slack(cus) + kNumXcd * (ffn_dim / kSddBN);
-  sdd_layer_kernel<CfgB><<<static_cast<uint32_t>(std::max<int64_t>(tiles + slack, cus)), 64 * kSddWaves, 0, stream>>>(
+  const bool dsd_narrow = may_be_narrow(min_rows, d_model, kDsdWidestNarrow, cus);
+  auto* kernel = may_be_narrow(min_rows, ffn_dim, kSddWidestNarrow, cus) ? sdd_layer_kernel<CfgB, true>
+                                                                         : sdd_layer_kernel<CfgB, false>;
+  kernel<<<static_cast<uint32_t>(std::max<int64_t>(tiles + slack, cus)), 64 * kSddWaves, 0, stream>>>(
       static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w1), row_token, row_block_expert, row_offsets,
       tokens_per_expert, padded_offsets, static_cast<uint16_t*>(out), static_cast<int32_t>(num_tokens),
       static_cast<int32_t>(d_model), static_cast<int32_t>(ffn_dim), static_cast<int32_t>(num_experts),
       static_cast<int32_t>(max_row_blocks), apply_gelu, kTileGroup, force,
-      static_cast<int32_t>(std::min<int64_t>(dsd_grid, 2147483647)), cus / kNumXcd, static_cast<int32_t>(slack));
+      static_cast<int32_t>(std::min<int64_t>(dsd_grid, 2147483647)), dsd_narrow ? 1 : 0, cus / kNumXcd,
+      static_cast<int32_t>(slack));
   return check_launch("sdd_experts");
 }
 
 int dispatch_sdd_layer(const void* x, const void* w1, const int32_t* row_token, const int32_t* row_block_expert,
                        const int32_t* row_offsets, const int32_t* tokens_per_expert, const int32_t* padded_offsets,
                        void* out, int64_t num_tokens, int64_t d_model, int64_t ffn_dim, int64_t num_experts,
-                       int64_t max_row_blocks, int32_t apply_gelu, int32_t force, hipStream_t stream) {
+                       int64_t max_row_blocks, int64_t min_rows, int32_t apply_gelu, int32_t force,
+                       hipStream_t stream) {
   // The row-block tile is sb_sdd's for the shape (sdd_tile_for).
   if (sdd_tile_for(d_model, ffn_dim) == SddTile::kDeep)
     return launch_sdd_layer<SddDeepTile>(x, w1, row_token, row_block_expert, row_offsets, tokens_per_expert,
                                          padded_offsets, out, num_tokens, d_model, ffn_dim, num_experts,
-                                         max_row_blocks, apply_gelu, force, stream);
+                                         max_row_blocks, min_rows, apply_gelu, force, stream);
   return launch_sdd_layer<SddWideTile>(x, w1, row_token, row_block_expert, row_offsets, tokens_per_expert,
                                        padded_offsets, out, num_tokens, d_model, ffn_dim, num_experts, max_row_blocks,
-                                       apply_gelu, force, stream);
+                                       min_rows, apply_gelu, force, stream);
 }
 
 int launch_sdd_pairs(const void* x, const void* w1, const int32_t* row_token, const int32_t* row_block_expert,
                      const int32_t* tokens_per_expert, const int32_t* padded_offsets, void* out, int64_t num_tokens,
-                     int64_t d_model, int64_t ffn_dim, int64_t num_experts, int64_t max_row_blocks, int32_t apply_gelu,
-                     int32_t force, hipStream_t stream) {
+                     int64_t d_model, int64_t ffn_dim, int64_t num_experts, int64_t max_row_blocks, int64_t min_rows,
+                     int32_t apply_gelu, int32_t force, hipStream_t stream) {
   if (!reduction_fits<SddPairTile>(d_model) || !reduction_fits<SddNarrowTile>(d_model) ||
       !reduction_fits<SddNarrowHalfTile>(d_model))
     return fail(SB_ERR_INVALID, "sdd_experts: D (%lld) is not a whole number of the tiles' K steps",
@@ -634,19 +649,22 @@ int launch_sdd_pairs(const void* x, const void* w1, const int32_t* row_token, co
   const int64_t grid =
       int64_t{kNumXcd} *
       (int64_t{pair_units_per_xcd(static_cast<int>(max_row_blocks))} * (ffn_dim / SddPairTile::BN) + cus_per_xcd / 2);
-  sdd_pair_kernel<SddPairTile, SddNarrowTile, SddNarrowHalfTile>
-      <<<static_cast<uint32_t>(std::max<int64_t>(grid, cus)), SddPairTile::kThreads, 0, stream>>>(
-          static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w1), row_token, row_block_expert,
-          tokens_per_expert, padded_offsets, static_cast<uint16_t*>(out), static_cast<int32_t>(num_tokens),
-          static_cast<int32_t>(d_model), static_cast<int32_t>(ffn_dim), static_cast<int32_t>(num_experts),
-          static_cast<int32_t>(max_row_blocks), apply_gelu, force, cus_per_xcd);
+  const bool dsd_narrow = may_be_narrow(min_rows, d_model, kDsdWidestNarrow, cus);
+  auto* kernel = may_be_narrow(min_rows, ffn_dim, kSddWidestNarrow, cus)
+                     ? sdd_pair_kernel<SddPairTile, SddNarrowTile, SddNarrowHalfTile, true>
+                     : sdd_pair_kernel<SddPairTile, SddNarrowTile, SddNarrowHalfTile, false>;
+  kernel<<<static_cast<uint32_t>(std::max<int64_t>(grid, cus)), SddPairTile::kThreads, 0, stream>>>(
+      static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w1), row_token, row_block_expert,
+      tokens_per_expert, padded_offsets, static_cast<uint16_t*>(out), static_cast<int32_t>(num_tokens),
+      static_cast<int32_t>(d_model), static_cast<int32_t>(ffn_dim), static_cast<int32_t>(num_experts),
+      static_cast<int32_t>(max_row_blocks), apply_gelu, force, dsd_narrow ? 1 : 0, cus_per_xcd);
   return check_launch("sdd_experts");
 }
 
 template <class CfgB, int WAVES>
 int launch_dsd_layer(const void* h, const void* w2, const int32_t* tokens_per_expert, const int32_t* padded_offsets,
                      const int32_t* row_block_expert, void* out, int64_t max_row_blocks, int64_t num_experts,
-                     int64_t num_copies, int64_t ffn_dim, int64_t d_model, int32_t force, hipStream_t stream) {
+                     int64_t min_rows, int64_t ffn_dim, int64_t d_model, int32_t force, hipStream_t stream) {
   static_assert(CfgB::BN == 512 || CfgB::BN == 256, "row-block tile widths of dsd_layer_grid");
   if (!reduction_fits<CfgB>(ffn_dim) || !reduction_fits<DsdCfg<4, kDsdBN, WAVES, kDsdStages>>(ffn_dim))
     return fail(SB_ERR_INVALID, "dsd_experts: F (%lld) is not a whole number of the tiles' K steps",
@@ -657,7 +675,9 @@ int launch_dsd_layer(const void* h, const void* w2, const int32_t* tokens_per_ex
   int cus = 0;
   if (const int rc = device_cus(&cus)) return rc;
   const int64_t slack = split_tail_slack(cus);
-  dsd_layer_kernel<CfgB, WAVES><<<static_cast<uint32_t>(std::max<int64_t>(tiles + slack, cus)), 64 * WAVES, 0, stream>>>(
+  auto* kernel = may_be_narrow(min_rows, d_model, kDsdWidestNarrow, cus) ? dsd_layer_kernel<CfgB, WAVES, true>
+                                                                         : dsd_layer_kernel<CfgB, WAVES, false>;
+  kernel<<<static_cast<uint32_t>(std::max<int64_t>(tiles + slack, cus)), 64 * WAVES, 0, stream>>>(
       static_cast<const uint16_t*>(h), static_cast<const uint16_t*>(w2), tokens_per_expert, padded_offsets,
       row_block_expert, static_cast<uint16_t*>(out), h_bytes, static_cast<int32_t>(num_experts),
       static_cast<int32_t>(ffn_dim), static_cast<int32_t>(d_model), static_cast<int32_t>(max_row_blocks),
@@ -666,15 +686,11 @@ int launch_dsd_layer(const void* h, const void* w2, const int32_t* tokens_per_ex
 }
 
 }  // namespace
-}  // namespace sb
 
-using namespace sb;
-
-extern "C" int sb_sdd_experts(const void* x, const void* w1, const int32_t* row_token,
-                              const int32_t* row_block_expert, const int32_t* row_offsets,
-                              const int32_t* tokens_per_expert, const int32_t* padded_offsets, void* out,
-                              int64_t num_tokens, int64_t d_model, int64_t ffn_dim, int64_t num_experts,
-                              int64_t max_row_blocks, int32_t apply_gelu, void* stream) {
+int sdd_experts(const void* x, const void* w1, const int32_t* row_token, const int32_t* row_block_expert,
+                const int32_t* row_offsets, const int32_t* tokens_per_expert, const int32_t* padded_offsets, void* out,
+                int64_t num_tokens, int64_t d_model, int64_t ffn_dim, int64_t num_experts, int64_t max_row_blocks,
+                int64_t min_rows, int32_t apply_gelu, void* stream) {
   constexpr int64_t kI32Max = 2147483647;
   if (max_row_blocks < 0) return fail(SB_ERR_INVALID, "sdd_experts: negative row block count");
   if (max_row_blocks == 0) return clear_ok();
@@ -704,21 +720,20 @@ extern "C" int sb_sdd_experts(const void* x, const void* w1, const int32_t* row_
                   max_row_blocks, apply_gelu, stream);
   if (ffn_dim % kSddBN != 0) {
     const int rc = launch_sdd_pairs(x, w1, row_token, row_block_expert, tokens_per_expert, padded_offsets, out,
-                                    num_tokens, d_model, ffn_dim, num_experts, max_row_blocks, apply_gelu, force,
-                                    as_stream(stream));
+                                    num_tokens, d_model, ffn_dim, num_experts, max_row_blocks, min_rows, apply_gelu,
+                                    force, as_stream(stream));
     return rc ? rc : clear_ok();
   }
   const int rc = dispatch_sdd_layer(x, w1, row_token, row_block_expert, row_offsets, tokens_per_expert, padded_offsets,
-                                    out, num_tokens, d_model, ffn_dim, num_experts, max_row_blocks, apply_gelu, force,
-                                    as_stream(stream));
+                                    out, num_tokens, d_model, ffn_dim, num_experts, max_row_blocks, min_rows,
+                                    apply_gelu, force, as_stream(stream));
   return rc ? rc : clear_ok();
 }
 
-extern "C" int sb_dsd_experts(const void* h, const void* w2, const int32_t* tokens_per_expert,
-                              const int32_t* padded_offsets, const int32_t* row_block_expert,
-                              const int32_t* row_offsets, const int32_t* col_indices, void* out,
-                              int64_t max_row_blocks, int64_t num_experts, int64_t num_copies, int64_t ffn_dim,
-                              int64_t d_model, void* stream) {
+int dsd_experts(const void* h, const void* w2, const int32_t* tokens_per_expert, const int32_t* padded_offsets,
+                const int32_t* row_block_expert, const int32_t* row_offsets, const int32_t* col_indices, void* out,
+                int64_t max_row_blocks, int64_t num_experts, int64_t num_copies, int64_t min_rows, int64_t ffn_dim,
+                int64_t d_model, void* stream) {
   constexpr int64_t kI32Max = 2147483647;
   if (max_row_blocks < 0) return fail(SB_ERR_INVALID, "dsd_experts: negative row block count");
   if (max_row_blocks == 0) return clear_ok();
@@ -748,7 +763,7 @@ extern "C" int sb_dsd_experts(const void* h, const void* w2, const int32_t* toke
   // 128 x 256 when D % 512 != 0. The expert tiles take the same wave count.
   auto launch = [&](auto cfg, auto waves) {  // cfg: Tag<row-block config>
     return launch_dsd_layer<typename decltype(cfg)::type, decltype(waves)::value>(
-        h, w2, tokens_per_expert, padded_offsets, row_block_expert, out, max_row_blocks, num_experts, num_copies,
+        h, w2, tokens_per_expert, padded_offsets, row_block_expert, out, max_row_blocks, num_experts, min_rows,
         ffn_dim, d_model, force, s);
   };
   using W4 = std::integral_constant<int, 4>;
@@ -759,4 +774,27 @@ extern "C" int sb_dsd_experts(const void* h, const void* w2, const int32_t* toke
                       : (deep ? launch(Tag<DsdCfg<4, 256, 8, 4>>{}, W8{})
                               : launch(Tag<DsdCfg<4, 256, 4, 4>>{}, W4{}));
   return rc ? rc : clear_ok();
+}
+
+}  // namespace sb
+
+using namespace sb;
+
+// A layout alone does not say how many rows are routed.
+extern "C" int sb_sdd_experts(const void* x, const void* w1, const int32_t* row_token,
+                              const int32_t* row_block_expert, const int32_t* row_offsets,
+                              const int32_t* tokens_per_expert, const int32_t* padded_offsets, void* out,
+                              int64_t num_tokens, int64_t d_model, int64_t ffn_dim, int64_t num_experts,
+                              int64_t max_row_blocks, int32_t apply_gelu, void* stream) {
+  return sdd_experts(x, w1, row_token, row_block_expert, row_offsets, tokens_per_expert, padded_offsets, out,
+                     num_tokens, d_model, ffn_dim, num_experts, max_row_blocks, 0, apply_gelu, stream);
+}
+
+extern "C" int sb_dsd_experts(const void* h, const void* w2, const int32_t* tokens_per_expert,
+                              const int32_t* padded_offsets, const int32_t* row_block_expert,
+                              const int32_t* row_offsets, const int32_t* col_indices, void* out,
+                              int64_t max_row_blocks, int64_t num_experts, int64_t num_copies, int64_t ffn_dim,
+                              int64_t d_model, void* stream) {
+  return dsd_experts(h, w2, tokens_per_expert, padded_offsets, row_block_expert, row_offsets, col_indices, out,
+                     max_row_blocks, num_experts, num_copies, 0, ffn_dim, d_model, stream);
 }

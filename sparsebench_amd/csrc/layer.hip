@@ -112,13 +112,14 @@ int check_workspace(const void* workspace, int64_t workspace_bytes, int64_t need
 }
 
 int run_sdd_dsd(const LayerBuffers& b, const void* x, const void* w1, const void* w2, int64_t num_tokens,
-                int64_t num_copies, int64_t d_model, int64_t ffn_dim, int64_t num_experts, void* stream) {
-  if (int rc = sb_sdd_experts(x, w1, b.row_token, b.row_block_expert, b.row_offsets, b.tokens_per_expert,
-                              b.padded_offsets, b.h, num_tokens, d_model, ffn_dim, num_experts, b.max_row_blocks, 1,
-                              stream))
+                int64_t num_copies, int64_t min_rows, int64_t d_model, int64_t ffn_dim, int64_t num_experts,
+                void* stream) {
+  if (int rc = sdd_experts(x, w1, b.row_token, b.row_block_expert, b.row_offsets, b.tokens_per_expert,
+                           b.padded_offsets, b.h, num_tokens, d_model, ffn_dim, num_experts, b.max_row_blocks, min_rows,
+                           1, stream))
     return rc;
-  return sb_dsd_experts(b.h, w2, b.tokens_per_expert, b.padded_offsets, b.row_block_expert, b.row_offsets,
-                        b.col_indices, b.y, b.max_row_blocks, num_experts, num_copies, ffn_dim, d_model, stream);
+  return dsd_experts(b.h, w2, b.tokens_per_expert, b.padded_offsets, b.row_block_expert, b.row_offsets, b.col_indices,
+                     b.y, b.max_row_blocks, num_experts, num_copies, min_rows, ffn_dim, d_model, stream);
 }
 
 }  // namespace
@@ -160,7 +161,9 @@ extern "C" int sb_layer(const void* x, const void* expert_idx, int32_t idx_is_i6
                           static_cast<int32_t>(kBlock), valid_tokens, b.counts, l.tokens_per_expert, l.padded_offsets,
                           l.row_token, l.copy_row, l.row_block_expert, l.row_offsets, l.col_indices, l.error, stream))
     return rc;
-  if (int rc = run_sdd_dsd(l, x, w1, w2, num_tokens, n, d_model, ffn_dim, num_experts, stream)) return rc;
+  // All copies are routed, but for ids out of range (an error) and tokens from *valid_tokens on.
+  const int64_t min_rows = valid_tokens ? 0 : n;
+  if (int rc = run_sdd_dsd(l, x, w1, w2, num_tokens, n, min_rows, d_model, ffn_dim, num_experts, stream)) return rc;
   return sb_combine(l.y, l.copy_row, gates, gate_dtype, out, num_tokens, k, d_model, l.max_row_blocks * kBlock,
                     valid_tokens, stream);
 }
@@ -184,7 +187,9 @@ extern "C" int sb_layer_assigned(const void* x, const void* token_of_copy, int32
   if (int rc = sb_token_csr(token_of_copy, token_is_i64, l.copy_row, num_copies, num_tokens, b.token_offsets,
                             b.token_copies, stream))
     return rc;
-  if (int rc = run_sdd_dsd(l, x, w1, w2, num_tokens, num_copies, d_model, ffn_dim, num_experts, stream)) return rc;
+  const int64_t min_rows = valid_tokens ? 0 : num_copies;
+  if (int rc = run_sdd_dsd(l, x, w1, w2, num_tokens, num_copies, min_rows, d_model, ffn_dim, num_experts, stream))
+    return rc;
   return sb_combine_assigned(l.y, l.copy_row, weights, weight_dtype, b.token_offsets, b.token_copies, out, num_tokens,
                              d_model, l.max_row_blocks * kBlock, valid_tokens, stream);
 }
@@ -203,7 +208,10 @@ extern "C" int sb_layer_rounded(const void* x, const float* scores, const void* 
                                  l.padded_offsets, l.row_token, l.copy_row, l.row_block_expert, l.row_offsets,
                                  l.col_indices, l.error, stream))
     return rc;
-  if (int rc = run_sdd_dsd(l, x, w1, w2, num_tokens, b.capacity, d_model, ffn_dim, num_experts, stream)) return rc;
+  // Rounding, to the tile or the largest multiple of it in T, takes less than a tile from an expert.
+  const int64_t min_rows = num_tokens * k - static_cast<int64_t>(num_experts) * (tile - 1);
+  if (int rc = run_sdd_dsd(l, x, w1, w2, num_tokens, b.capacity, min_rows, d_model, ffn_dim, num_experts, stream))
+    return rc;
   return sb_combine_assigned(l.y, l.copy_row, b.weight_of_copy, SB_DTYPE_F32, b.token_offsets, nullptr, out,
                              num_tokens, d_model, l.max_row_blocks * kBlock, nullptr, stream);
 }

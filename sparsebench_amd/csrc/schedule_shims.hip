@@ -2,8 +2,9 @@
 // over the same __host__ __device__ functions the kernels call
 // (common.hpp: xcd_remap, split_tail, split_tail_slack, tile_coords;
 // expert_chunks.hpp: balanced_chunk_tile, lpt_group_tile, pair_units_per_xcd,
-// pair_tile_for, narrow_width, narrow_tile_for), so tests/test_tile_schedules.py checks the compiled
-// mappings themselves. Part of the tool library (libsparsebench_probe.so),
+// pair_tile_for, narrow_width, may_be_narrow, narrow_tile_for), so
+// tests/test_tile_schedules.py and tests/test_narrow_tiles.py check the
+// compiled mappings themselves. Part of the tool library (libsparsebench_probe.so),
 // not of libsparsebench_hip.so's C ABI. No kernel runs.
 
 #include "expert_chunks.hpp"
@@ -44,6 +45,10 @@ extern "C" void sbt_lpt_group_tile(int local, int groups, int slices, uint32_t b
 
 extern "C" int sbt_narrow_width(int live_rb, int columns, int widest, int cus) {
   return narrow_width(live_rb, columns, widest, cus);
+}
+
+extern "C" int sbt_may_be_narrow(int64_t min_rows, int64_t columns, int widest, int cus) {
+  return may_be_narrow(min_rows, columns, widest, cus) ? 1 : 0;
 }
 
 extern "C" void sbt_narrow_tile_for(int bid, int live_rb, int slices, int* rb, int* slice) {

@@ -90,6 +90,26 @@ def test_same_bits_as_the_stages(form: str) -> None:
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("routed", ["all", "few"])
+@pytest.mark.parametrize(("t", "e", "d", "f"), [
+    (2048, 8, 1280, 4096),  # neither stage can be narrow
+    (2048, 8, 512, 4096), (512, 2, 8192, 512),  # the SDD cannot; the DSD cannot
+    (1024, 4, 2304, 8192), (512, 2, 8192, 8192),  # the same with the DSD's 8 waves: neither; the DSD
+    (2048, 8, 1280, 4352),  # F % 512 != 0
+])
+def test_instances_without_narrow_tiles_same_bits(t: int, e: int, d: int, f: int, routed: str) -> None:
+    # The one call launches its stages without narrow tiles where 2 T routed copies rule them out; stage by stage
+    # they are always there. With most ids out of range few row blocks live after all: the same rows still.
+    from sparsebench_amd.moe import moe_forward
+
+    x, idx, gates, w1, w2 = layer(t, e, d, f)
+    if routed == "few":
+        idx[3:] = e
+    got = moe_forward(x, idx, gates, w1, w2)
+    assert torch.equal(got, moe_forward(x, idx, gates, w1, w2, mark=staged))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("index", [torch.int32, torch.int64])
 def test_assigned_and_rounded_same_bits(index: torch.dtype) -> None:
     from sparsebench_amd.moe import moe_forward_assigned, moe_forward_rounded

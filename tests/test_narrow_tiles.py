@@ -52,6 +52,17 @@ def test_width_rule_and_tile_order(sched, columns: int, widest: int) -> None:
         assert sorted(seen) == [(r, s) for r in range(live) for s in range(slices)]
 
 
+@pytest.mark.parametrize("columns", [256, 768, 2048, 4352, 14336])
+@pytest.mark.parametrize("widest", [128, 256])
+def test_instances_without_narrow_tiles(sched, columns: int, widest: int) -> None:
+    # Launched only when no layout of at least min_rows rows would take a narrow tile; always launched then.
+    sched.sbt_may_be_narrow.argtypes = [ctypes.c_int64, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
+    for min_rows in [-5, 0, 1, 128, 129, 1000, 2047, 2048, 2049, 32768, 32769, 10**6, 2**40]:
+        live = max(0, -(-min_rows // 128))
+        widths = [sched.sbt_narrow_width(n, columns, widest, CUS) for n in range(live, CUS + 2)]
+        assert bool(sched.sbt_may_be_narrow(min_rows, columns, widest, CUS)) == (live == 0 or any(widths))
+
+
 SINGLE = [1, 33, 0, 70, 127]  # one row block each: 1, 2, 3 and 4 row groups
 CASES = {
     # name: (rows per expert, D, F); the stages' widths follow from row blocks x columns
