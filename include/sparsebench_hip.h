@@ -115,6 +115,14 @@ int sb_dsd(const void* blocks, const void* w, const int32_t* row_offsets, const 
            int64_t nnz, int64_t w_rows, int64_t num_row_blocks, int64_t block_size, int64_t d_model,
            int32_t zero_dead_rows, void* stream);
 
+/* sb_dsd, told that the arrays are a routing layout (sb_routing's and its
+ * variants'), where an expert's row blocks have the same block columns: with
+ * block size 64 it may then run them in pairs. The results are sb_dsd's for
+ * any BSR; others are only slower this way. */
+int sb_dsd_routed(const void* blocks, const void* w, const int32_t* row_offsets, const int32_t* col_indices, void* out,
+                  int64_t nnz, int64_t w_rows, int64_t num_row_blocks, int64_t block_size, int64_t d_model,
+                  int32_t zero_dead_rows, void* stream);
+
 /* Replace the SDD and DSD stages of moe_forward (sparsebench/moe.py:46-48:
  * spmm.sdd then spmm.dsd version 5 on route_device's layout). Each call
  * enqueues one kernel whose workgroups choose, on the GPU and all alike from

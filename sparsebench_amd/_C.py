@@ -188,13 +188,17 @@ def sdd_cuda(
 
 
 def dsd_cuda(
-    blocks: torch.Tensor, w: torch.Tensor, row_offsets: torch.Tensor, col_indices: torch.Tensor, version: int
+    blocks: torch.Tensor, w: torch.Tensor, row_offsets: torch.Tensor, col_indices: torch.Tensor, version: int,
+    routed: bool = False,
 ) -> torch.Tensor:
     """out [(len(row_offsets)-1)*bs, D] bf16 = BSR(blocks, row_offsets, col_indices) @ w.
 
     Every version code of the reference is accepted and gives the same
     results; codes 1, 2, 21, 3, 31 write dead row blocks as zeros, codes 4,
     41, 5 leave them unwritten, and 5 needs block size 128 and D % 256 == 0.
+
+    routed (this build's extension): the arrays are a routing layout, so the
+    kernel may take its row blocks in pairs; the results are the same.
     """
     if not (blocks.is_cuda and w.is_cuda):
         _fail("blocks and w must be CUDA tensors")
@@ -239,7 +243,8 @@ def dsd_cuda(
         _fail(f"unknown dsd version {version}")
     if version == 5 and (bs != 128 or d_model % 256):
         _fail(f"dsd v5 needs block size 128 and D a multiple of 256, got block size {bs}, D {d_model}")
-    check(lib().sb_dsd(
+    launch = lib().sb_dsd_routed if routed else lib().sb_dsd
+    check(launch(
         blocks.data_ptr(), w.data_ptr(), row_offsets.data_ptr(), col_indices.data_ptr(), out.data_ptr(),
         blocks.shape[0], w.shape[0], num_row_blocks, bs, d_model, 1 if _DSD_VERSIONS[version] else 0,
         stream_of(w.device),

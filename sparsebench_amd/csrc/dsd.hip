@@ -85,51 +85,18 @@ using DsdMid = DmaCfg<BM, 256, 64, 3, 2, 4, 0, 2, 3>;
 template <int BM>
 using DsdNarrow = DmaCfg<BM, 128, 64, 3, 2, 2, 0, 2, 5>;
 
-template <class... Args>
-int dispatch_dsd_128(int64_t d_model, int64_t row_k, int64_t num_row_blocks, int cus, Args... args) {
-  switch (fit_width(num_row_blocks, d_model, cus)) {
-    case 512: return row_k >= 8192 ? launch_dsd<DsdDeep<128>>(args...) : launch_dsd<DsdWide<128>>(args...);
-    case 256: return launch_dsd<DsdMid<128>>(args...);
-    default: return launch_dsd<DsdNarrow<128>>(args...);
+template <int BM, class... Args>
+int launch_dsd_form(const DsdForm& form, Args... args) {
+  switch (form.width) {
+    case 512: return form.deep ? launch_dsd<DsdDeep<BM>>(args...) : launch_dsd<DsdWide<BM>>(args...);
+    case 256: return launch_dsd<DsdMid<BM>>(args...);
+    default: return launch_dsd<DsdNarrow<BM>>(args...);
   }
 }
 
-// Block size 64: row blocks one by one, or in pairs (dsd_pair_tile). A
-// routing layout of E experts has about (row blocks + E) / 2 tile rows in
-// pairs: the pairs, and row blocks alone, which cost a whole tile, at every
-// second expert's end. Pairs are taken when they let 512-wide tiles that leave
-// CUs idle become 256-wide ones (at least 4 row blocks an expert), or when
-// there are more tiles than CUs and at least 8 row blocks an expert. F = 2048,
-// E = 16, one by one against pairs: D = 1024, 79 row blocks 46 against 38 us;
-// D = 1024, 271 row blocks 127 against 107; but D = 4096, 79 row blocks 138
-// against 153, D = 512 (256 and 128 wide) 29 against 44, and with 3 row blocks
-// an expert (D = 1024, F = 4096, E = 64) 174 against 188.
-template <class... Args>
-int dispatch_dsd_64(int64_t d_model, int64_t row_k, int64_t w_rows, int64_t num_row_blocks, int cus, Args... args) {
-  const int64_t experts = row_k > 0 ? w_rows / row_k : num_row_blocks;
-  const int single = fit_width(num_row_blocks, d_model, cus);
-  const int paired = fit_width((num_row_blocks + experts) / 2, d_model, cus);
-  const bool narrower = single == 512 && paired == 256 && num_row_blocks >= 4 * experts;
-  const bool many = num_row_blocks * (d_model / single) > cus && num_row_blocks >= 8 * experts;
-  if (row_k < int64_t{64} * kMaxPairBlocks && paired >= 256 && (narrower || many)) {
-    if (paired == 256) return launch_dsd_pairs<DsdMid<128>>(args...);
-    return row_k >= 8192 ? launch_dsd_pairs<DsdDeep<128>>(args...) : launch_dsd_pairs<DsdWide<128>>(args...);
-  }
-  switch (single) {
-    case 512: return row_k >= 8192 ? launch_dsd<DsdDeep<64>>(args...) : launch_dsd<DsdWide<64>>(args...);
-    case 256: return launch_dsd<DsdMid<64>>(args...);
-    default: return launch_dsd<DsdNarrow<64>>(args...);
-  }
-}
-
-}  // namespace
-}  // namespace sb
-
-using namespace sb;
-
-extern "C" int sb_dsd(const void* blocks, const void* w, const int32_t* row_offsets, const int32_t* col_indices,
-                      void* out, int64_t nnz, int64_t w_rows, int64_t num_row_blocks, int64_t block_size,
-                      int64_t d_model, int32_t zero_dead_rows, void* stream) {
+int dsd(const void* blocks, const void* w, const int32_t* row_offsets, const int32_t* col_indices, void* out,
+        int64_t nnz, int64_t w_rows, int64_t num_row_blocks, int64_t block_size, int64_t d_model,
+        int32_t zero_dead_rows, bool routed, void* stream) {
   constexpr int64_t kI32Max = 2147483647;
   if (block_size != 64 && block_size != 128)
     return fail(SB_ERR_INVALID, "block size must be 64 or 128, got %lld", static_cast<long long>(block_size));
@@ -146,15 +113,36 @@ extern "C" int sb_dsd(const void* blocks, const void* w, const int32_t* row_offs
   if (!blocks || !w || !row_offsets || !col_indices || !out) return fail(SB_ERR_INVALID, "dsd: null buffer");
   if (!aligned16(blocks) || !aligned16(w) || !aligned16(out))
     return fail(SB_ERR_INVALID, "blocks and w must be 16-byte aligned");
-  // The reduction depth per row block, from the buffer shape (nnz /
-  // num_row_blocks blocks per row), picks the deep-K tile.
-  const int64_t row_k = nnz / num_row_blocks * block_size;
   const hipStream_t s = as_stream(stream);
   int cus = 0;
   if (const int rc = device_cus(&cus)) return rc;
-  if (block_size == 128)
-    return dispatch_dsd_128(d_model, row_k, num_row_blocks, cus, blocks, w, row_offsets, col_indices, out, nnz, w_rows,
-                            num_row_blocks, d_model, zero_dead_rows, s);
-  return dispatch_dsd_64(d_model, row_k, w_rows, num_row_blocks, cus, blocks, w, row_offsets, col_indices, out, nnz,
-                         w_rows, num_row_blocks, d_model, zero_dead_rows, s);
+  const DsdForm form = dsd_form(block_size, nnz, w_rows, num_row_blocks, d_model, routed, cus);
+  auto with = [&](auto launch) {
+    return launch(blocks, w, row_offsets, col_indices, out, nnz, w_rows, num_row_blocks, d_model, zero_dead_rows, s);
+  };
+  if (block_size == 128) return with([&](auto... args) { return launch_dsd_form<128>(form, args...); });
+  if (!form.paired) return with([&](auto... args) { return launch_dsd_form<64>(form, args...); });
+  return with([&](auto... args) {
+    if (form.width == 256) return launch_dsd_pairs<DsdMid<128>>(args...);
+    return form.deep ? launch_dsd_pairs<DsdDeep<128>>(args...) : launch_dsd_pairs<DsdWide<128>>(args...);
+  });
+}
+
+}  // namespace
+}  // namespace sb
+
+using namespace sb;
+
+extern "C" int sb_dsd(const void* blocks, const void* w, const int32_t* row_offsets, const int32_t* col_indices,
+                      void* out, int64_t nnz, int64_t w_rows, int64_t num_row_blocks, int64_t block_size,
+                      int64_t d_model, int32_t zero_dead_rows, void* stream) {
+  return dsd(blocks, w, row_offsets, col_indices, out, nnz, w_rows, num_row_blocks, block_size, d_model,
+             zero_dead_rows, false, stream);
+}
+
+extern "C" int sb_dsd_routed(const void* blocks, const void* w, const int32_t* row_offsets, const int32_t* col_indices,
+                             void* out, int64_t nnz, int64_t w_rows, int64_t num_row_blocks, int64_t block_size,
+                             int64_t d_model, int32_t zero_dead_rows, void* stream) {
+  return dsd(blocks, w, row_offsets, col_indices, out, nnz, w_rows, num_row_blocks, block_size, d_model,
+             zero_dead_rows, true, stream);
 }

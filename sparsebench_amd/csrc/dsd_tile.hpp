@@ -230,4 +230,43 @@ __device__ __forceinline__ void dsd_pair_tile(uint8_t* __restrict__ lds, int bid
   });
 }
 
+// Which tiles sb_dsd runs: `width` columns (fit_width), deep = the 512-wide
+// ones' form for a reduction of at least 8192, paired = block size 64 with the
+// row blocks in pairs (dsd_pair_tile).
+struct DsdForm {
+  int width;
+  bool paired, deep;
+};
+
+// Block size 64: row blocks one by one, or in pairs. A routing layout
+// (`routed`) of E experts has about (row blocks + E) / 2 tile rows in pairs:
+// the pairs, and row blocks alone, which cost a whole tile, at every second
+// expert's end. Pairs are taken when they let 512-wide tiles that leave CUs
+// idle become 256-wide ones (at least 4 row blocks an expert), or when there
+// are more tiles than CUs and at least 8 row blocks an expert. F = 2048,
+// E = 16, one by one against pairs: D = 1024, 79 row blocks 46 against 38 us;
+// D = 1024, 271 row blocks 127 against 107; but D = 4096, 79 row blocks 138
+// against 153, D = 512 (256 and 128 wide) 29 against 44, and with 3 row blocks
+// an expert (D = 1024, F = 4096, E = 64) 174 against 188.
+// Of any other BSR the neighbours' columns differ, and every row block would
+// cost a whole tile for its half: none in pairs (64 column blocks, half of
+// them in each row: 256 row blocks, D = 1024 129 one by one against 147 us in
+// pairs; 64, D = 4096 145 against 160; 16 column blocks, 40 row blocks,
+// D = 8192 54 against 67).
+inline DsdForm dsd_form(int64_t block_size, int64_t nnz, int64_t w_rows, int64_t num_row_blocks, int64_t d_model,
+                        bool routed, int cus) {
+  // The reduction depth per row block, from the buffer shape (nnz /
+  // num_row_blocks blocks per row).
+  const int64_t row_k = nnz / num_row_blocks * block_size;
+  const bool deep = row_k >= 8192;
+  const int single = fit_width(num_row_blocks, d_model, cus);
+  if (block_size != 64 || !routed || row_k <= 0 || row_k >= int64_t{64} * kMaxPairBlocks) return {single, false, deep};
+  const int64_t experts = w_rows / row_k;
+  const int paired = fit_width((num_row_blocks + experts) / 2, d_model, cus);
+  const bool narrower = single == 512 && paired == 256 && num_row_blocks >= 4 * experts;
+  const bool many = num_row_blocks * (d_model / single) > cus && num_row_blocks >= 8 * experts;
+  if (paired >= 256 && (narrower || many)) return {paired, true, deep};
+  return {single, false, deep};
+}
+
 }  // namespace sb

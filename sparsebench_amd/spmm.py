@@ -23,7 +23,7 @@ def dsd(
     bs = topo.block_size
     if blocks.dim() != 3 or blocks.shape[1:] != (bs, bs):
         raise ValueError(f"blocks must be [nnz, {bs}, {bs}] for this topology, got {tuple(blocks.shape)}")
-    return _C.dsd_cuda(blocks, w2_cat, topo.row_offsets, topo.col_indices, version)
+    return _C.dsd_cuda(blocks, w2_cat, topo.row_offsets, topo.col_indices, version, routed=True)
 
 
 def sdd(x: torch.Tensor, w1: torch.Tensor, topo: Topology | DeviceTopology, gelu: bool = True) -> torch.Tensor:

@@ -40,15 +40,17 @@ def test_block_64_against_oracle(counts: list[int], d: int, f: int) -> None:
     w = torch.randn(e * f, d, generator=g).bfloat16()
     dead = 3
     offsets = torch.cat([torch.as_tensor(lay.row_offsets), torch.full((dead,), int(lay.row_offsets[-1]))]).int()
-    out = _C.dsd_cuda(blocks.cuda(), w.cuda(), offsets.cuda(), torch.as_tensor(lay.col_indices).cuda(), 1)
+    out = _C.dsd_cuda(blocks.cuda(), w.cuda(), offsets.cuda(), torch.as_tensor(lay.col_indices).cuda(), 1, routed=True)
     torch.testing.assert_close(out[: lay.num_rows].float().cpu(), dsd_rows(blocks.float(), w.float(), lay), **TOL)
     assert torch.all(out[lay.num_rows:] == 0)
 
 
+@pytest.mark.parametrize("routed", [False, True])
 @pytest.mark.parametrize("version", [1, 4])
-def test_block_64_any_bsr(version: int) -> None:
+def test_block_64_any_bsr(version: int, routed: bool) -> None:
     # Not a routing layout: block counts and columns differ from row to row, in an order of their own, some repeated,
-    # some out of w's range (they add nothing); 41 row blocks over one "expert" take the pairs.
+    # some out of w's range (they add nothing); 41 row blocks over one "expert" take the pairs
+    # when they are said to be a routing layout's.
     from sparsebench_amd import _C
 
     rng = np.random.default_rng(5)
@@ -67,7 +69,8 @@ def test_block_64_any_bsr(version: int) -> None:
     g = torch.Generator().manual_seed(2)
     blocks = (torch.randn(flat.size, 64, 64, generator=g) / 20).bfloat16()
     w = torch.randn(col_blocks * 64, d, generator=g).bfloat16()
-    out = _C.dsd_cuda(blocks.cuda(), w.cuda(), torch.as_tensor(offsets).cuda(), torch.as_tensor(flat).cuda(), version)
+    out = _C.dsd_cuda(blocks.cuda(), w.cuda(), torch.as_tensor(offsets).cuda(), torch.as_tensor(flat).cuda(), version,
+                      routed=routed)
     wide = torch.cat([w.float(), torch.zeros(64, d)])  # the block past w
     for r in range(rows):
         if not cols[r] and version == 4:
@@ -82,9 +85,7 @@ def test_block_64_any_bsr(version: int) -> None:
 def test_block_64_long_rows_among_short_ones(version: int) -> None:
     # Row blocks of 65536 blocks (columns repeated), more than a pair takes, as the first and the second of theirs,
     # in a layout that takes pairs. Small whole numbers: every sum is exact, up to the rounding of the result.
-    from types import SimpleNamespace
-
-    from sparsebench_amd.spmm import dsd
+    from sparsebench_amd import _C
 
     d, col_blocks, rows, long = 512, 8, 1024, {0, 3}
     counts = torch.tensor([65536 if r in long else 8 for r in range(rows)])
@@ -93,9 +94,8 @@ def test_block_64_long_rows_among_short_ones(version: int) -> None:
     g = torch.Generator(device="cuda").manual_seed(4)
     blocks = torch.randint(-1, 2, (nnz, 64, 64), generator=g, device="cuda", dtype=torch.int8).bfloat16()
     w = torch.randint(-1, 2, (col_blocks * 64, d), generator=g, device="cuda", dtype=torch.int8).bfloat16()
-    topo = SimpleNamespace(block_size=64, row_offsets=offsets.int().cuda(),
-                           col_indices=(torch.arange(nnz, device="cuda") % col_blocks).int())
-    out = dsd(blocks, w, topo, version)
+    cols = (torch.arange(nnz, device="cuda") % col_blocks).int()
+    out = _C.dsd_cuda(blocks, w, offsets.int().cuda(), cols, version, routed=True)
     for r in (0, 1, 2, 3, 4, 5, rows - 1):
         own = blocks[offsets[r]: offsets[r + 1]].view(-1, col_blocks, 64, 64).sum(0, dtype=torch.float32)
         want = own.permute(1, 0, 2).reshape(64, -1).double() @ w.double()
