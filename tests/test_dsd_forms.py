@@ -25,7 +25,7 @@ def form():
 
 
 # (row blocks, block columns, D, share of the blocks held)
-RANDOM = [(256, 64, 1024, 0.5), (64, 64, 4096, 0.5), (128, 64, 2048, 0.25), (512, 128, 512, 0.1), (40, 16, 8192, 0.5),
+RANDOM = [(300, 64, 1024, 0.5), (96, 64, 4096, 0.5), (150, 64, 2048, 0.25), (640, 128, 512, 0.1), (40, 16, 8192, 0.5),
           (1024, 8, 512, 16)]
 
 
@@ -35,6 +35,19 @@ def test_pairs_only_for_routing_layouts(form, rb: int, cols: int, d: int, share:
     assert form(64, nnz, w_rows, rb, d, 1, CUS) & 1  # by size alone they would take pairs
     assert not form(64, nnz, w_rows, rb, d, 0, CUS) & 1
     assert not form(128, nnz, w_rows * 2, rb, d, 1, CUS) & 1
+
+
+@pytest.mark.parametrize(("e", "d", "rows", "paired"), [
+    # rows: row blocks that hold rows; one expert's odd one out and the worst case add up to E more
+    (16, 1024, 63, True), (2, 768, 104, True), (1, 512, 158, True),     # the pairs leave three CUs of eight
+    (4, 1536, 66, False), (2, 768, 158, False), (16, 512, 400, False),  # one round, nearly full
+    (16, 1024, 122, False),                                             # one by one may be one round
+    (20, 1024, 80, False),                                              # many row blocks alone
+    (2, 512, 510, False), (16, 512, 545, True), (16, 1024, 290, True),  # just over one round, or surely more
+])
+def test_pairs_leave_room_for_row_blocks_alone(form, e: int, d: int, rows: int, paired: bool) -> None:
+    ffn, rb = 2048, rows + e
+    assert bool(form(64, rb * (ffn // 64), e * ffn, rb, d, 1, CUS) & 1) == paired
 
 
 @pytest.mark.parametrize("rb", [1, 7, 64, 1000])
