@@ -178,14 +178,42 @@ __global__ void __launch_bounds__(kTopkThreads)
       chunk_counts[static_cast<int64_t>(blockIdx.x) * num_experts + e] = hist[e];
 }
 
+// A lane's KMAX best (score, expert), sorted by (score desc, expert asc), of
+// which the first k are kept.
+template <int KMAX>
+struct BestK {
+  float bv[KMAX];
+  int bi[KMAX];
+  int k;
+  __device__ __forceinline__ explicit BestK(int kept) : k(kept) {
+#pragma unroll
+    for (int j = 0; j < KMAX; ++j) {
+      bv[j] = 0.0f;
+      bi[j] = 0x7fffffff;  // empty
+    }
+  }
+  __device__ __forceinline__ void offer(float v, int e) {
+#pragma unroll
+    for (int j = 0; j < KMAX; ++j) {  // selects, not branches: the lanes disagree at every step
+      const bool in = (j < k) & ((bi[j] == 0x7fffffff) | (v > bv[j]) | ((v == bv[j]) & (e < bi[j])));
+      const float tv = in ? bv[j] : v;
+      const int ti = in ? bi[j] : e;
+      bv[j] = in ? v : bv[j];
+      bi[j] = in ? e : bi[j];
+      v = tv;
+      e = ti;
+    }
+  }
+};
+
 // Top-k with one lane per token (64 tokens per workgroup, the same chunking
 // as router_topk_kernel). The workgroup's four waves read the scores a tile of
 // 64 tokens x up to kLaneTile experts at a time into LDS, whole rows of a
 // token side by side, and write the shifted scores from there; the first
 // wave's lanes walk their tokens' rows in the tile in expert order and keep
-// the KMAX best in registers, sorted by (score desc, expert asc): each new
-// (score, e) is bubbled in with compare-and-swap steps, so an equal score
-// behind an earlier expert stays behind it. No lane talks to another, and the
+// the KMAX best in registers (BestK): each new (score, e) is bubbled in with
+// compare-and-swap steps, so an equal score behind an earlier expert stays
+// behind it. No lane talks to another, and the
 // expert-major stores of the shifted scores are 64 consecutive tokens per
 // instruction. The outputs are those of router_topk_kernel. Bound by the
 // latency of its loads: with each lane reading its own row from memory,
@@ -230,25 +258,7 @@ __global__ void __launch_bounds__(kTopkThreads)
     __syncthreads();
   };
 
-  float bv[KMAX];
-  int bi[KMAX];
-#pragma unroll
-  for (int j = 0; j < KMAX; ++j) {
-    bv[j] = 0.0f;
-    bi[j] = 0x7fffffff;  // empty
-  }
-  auto offer = [&](float v, int e) {
-#pragma unroll
-    for (int j = 0; j < KMAX; ++j) {  // selects, not branches: the lanes disagree at every step
-      const bool in = (j < k) & ((bi[j] == 0x7fffffff) | (v > bv[j]) | ((v == bv[j]) & (e < bi[j])));
-      const float tv = in ? bv[j] : v;
-      const int ti = in ? bi[j] : e;
-      bv[j] = in ? v : bv[j];
-      bi[j] = in ? e : bi[j];
-      v = tv;
-      e = ti;
-    }
-  };
+  BestK<KMAX> best(k);
   for (int e0 = 0; e0 < num_experts; e0 += kLaneTile) {
     const int width = min(kLaneTile, num_experts - e0);
     load_tile(e0, width);
@@ -260,26 +270,26 @@ __global__ void __launch_bounds__(kTopkThreads)
 #pragma unroll
         for (int u = 0; u < kBatch; ++u) v[u] = tile[lane * (kLaneTile + 1) + e + u];
 #pragma unroll
-        for (int u = 0; u < kBatch; ++u) offer(v[u], e0 + e + u);
+        for (int u = 0; u < kBatch; ++u) best.offer(v[u], e0 + e + u);
       }
-      for (; e < width; ++e) offer(tile[lane * (kLaneTile + 1) + e], e0 + e);
+      for (; e < width; ++e) best.offer(tile[lane * (kLaneTile + 1) + e], e0 + e);
     }
   }
   if (wave == 0 && lane < tokens) {
     float total = 0.0f;
 #pragma unroll
     for (int j = 0; j < KMAX; ++j) {
-      if (j < k && bi[j] != 0x7fffffff) {
-        total += bv[j];  // in pick order
-        picked_bits[lane * words + (bi[j] >> 5)] |= 1u << (bi[j] & 31);
-        if (chunk_counts != nullptr) atomicAdd(&hist[bi[j]], 1);
-        if (top_idx != nullptr) top_idx[t * k + j] = bi[j];
+      if (j < k && best.bi[j] != 0x7fffffff) {
+        total += best.bv[j];  // in pick order
+        picked_bits[lane * words + (best.bi[j] >> 5)] |= 1u << (best.bi[j] & 31);
+        if (chunk_counts != nullptr) atomicAdd(&hist[best.bi[j]], 1);
+        if (top_idx != nullptr) top_idx[t * k + j] = best.bi[j];
       }
     }
     if (top_weight != nullptr)
 #pragma unroll
       for (int j = 0; j < KMAX; ++j)
-        if (j < k) top_weight[t * k + j] = bv[j] / total;
+        if (j < k) top_weight[t * k + j] = best.bv[j] / total;
   }
   __syncthreads();
   if (shifted != nullptr) {
@@ -297,6 +307,54 @@ __global__ void __launch_bounds__(kTopkThreads)
   if (chunk_counts != nullptr)
     for (int e = tid; e < num_experts; e += kTopkThreads)
       chunk_counts[static_cast<int64_t>(blockIdx.x) * num_experts + e] = hist[e];
+}
+
+// Top-k alone, each lane walking its token's own row from memory: for few
+// experts, whose rows the tiles' loads would leave mostly idle, and for so many
+// tokens that the waves hide the loads' latency, where the tiles' LDS keeps all
+// but a few waves off a CU. The outputs are those of router_topk_kernel.
+template <int KMAX>
+__global__ void __launch_bounds__(64)
+    router_topk_direct_kernel(const float* __restrict__ scores, int64_t num_tokens, int32_t num_experts, int32_t k,
+                              int32_t* __restrict__ top_idx, float* __restrict__ top_weight) {
+  const int64_t t = static_cast<int64_t>(blockIdx.x) * 64 + threadIdx.x;
+  if (t >= num_tokens) return;
+  const float* row = scores + t * num_experts;
+  BestK<KMAX> best(k);
+  int e = 0;
+  if ((num_experts & 3) == 0 && (reinterpret_cast<uintptr_t>(scores) & 15) == 0) {
+    for (; e + 16 <= num_experts; e += 16) {  // 16 scores (four 16-byte loads) in flight
+      float4 q[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) q[u] = *reinterpret_cast<const float4*>(row + e + 4 * u);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        best.offer(q[u].x, e + 4 * u);
+        best.offer(q[u].y, e + 4 * u + 1);
+        best.offer(q[u].z, e + 4 * u + 2);
+        best.offer(q[u].w, e + 4 * u + 3);
+      }
+    }
+    for (; e < num_experts; e += 4) {
+      const float4 q = *reinterpret_cast<const float4*>(row + e);
+      best.offer(q.x, e);
+      best.offer(q.y, e + 1);
+      best.offer(q.z, e + 2);
+      best.offer(q.w, e + 3);
+    }
+  }
+  for (; e < num_experts; ++e) best.offer(row[e], e);
+  float total = 0.0f;
+#pragma unroll
+  for (int j = 0; j < KMAX; ++j)
+    if (j < k) {
+      if (top_idx != nullptr) top_idx[t * k + j] = best.bi[j];
+      total += best.bv[j];  // in pick order
+    }
+  if (top_weight != nullptr)
+#pragma unroll
+    for (int j = 0; j < KMAX; ++j)
+      if (j < k) top_weight[t * k + j] = best.bv[j] / total;
 }
 
 // Inclusive scan over the lanes of one 1024-lane workgroup.
@@ -708,13 +766,27 @@ int launch_topk(const float* scores, int64_t num_tokens, int32_t num_experts, in
   const int kmax = k <= 1 ? 1 : k <= 2 ? 2 : k <= 4 ? 4 : k <= 8 ? 8 : 16;
   const int forced = test_hook(SB_HOOK_TOPK_KERNEL);
   if (forced == 2 || (forced != 1 && kmax * num_experts <= 8192)) {
-#define SB_TOPK_LANE(K) \
+    // Alone, the direct form for up to 8 experts (T = 4096, k = 2: E = 8 2.8
+    // against 3.8 us, E = 16 in tiles 4.0 and direct 4.2) and from 512 groups on
+    // (T = 131072, k = 2: E = 32 5.5 against 13.1; T = 32768, E = 64 7.0 in tiles,
+    // 10.8 direct), where a lane reads 16 bytes at a time or few at all
+    // (T = 300000, E = 129, k = 4 in tiles 124, direct 650).
+    const bool wide = num_experts % 4 == 0 && aligned16(scores);
+    const bool direct = shifted == nullptr && chunk_counts == nullptr &&
+                        (num_experts <= 8 || (groups > 512 && (wide || num_experts <= std::max(48, 8 * kmax))));
+    // Rows read 4 bytes at a time are read again and again from L1, which holds
+    // those of a few waves: LDS that the kernel does not use keeps a CU at 13
+    // (T = 300000, E = 45, k = 8 165 us without, 88 with).
+    const uint32_t waves_lds = wide || num_experts <= 8 ? 0 : 12 * 1024;
+#define SB_TOPK_LANE(K)                                                                                             \
+  if (direct) router_topk_direct_kernel<K><<<groups, 64, waves_lds, s>>>(scores, num_tokens, num_experts, k, top_idx, top_weight); \
+  else \
   router_topk_lane_kernel<K><<<groups, kTopkThreads, 0, s>>>(scores, num_tokens, num_experts, k, shifted, chunk_counts, top_idx, top_weight)
-    if (k <= 1) SB_TOPK_LANE(1);
-    else if (k <= 2) SB_TOPK_LANE(2);
-    else if (k <= 4) SB_TOPK_LANE(4);
-    else if (k <= 8) SB_TOPK_LANE(8);
-    else SB_TOPK_LANE(16);
+    if (k <= 1) { SB_TOPK_LANE(1); }
+    else if (k <= 2) { SB_TOPK_LANE(2); }
+    else if (k <= 4) { SB_TOPK_LANE(4); }
+    else if (k <= 8) { SB_TOPK_LANE(8); }
+    else { SB_TOPK_LANE(16); }
 #undef SB_TOPK_LANE
     return check_launch("router top-k");
   }

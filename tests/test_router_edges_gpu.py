@@ -41,3 +41,27 @@ def test_list_matches_oracle(t: int, e: int, k: int, tile: int, levels: int) -> 
     # copy_row and row_token name each other.
     rows = r.topology.copy_row.cpu().numpy()
     assert np.array_equal(r.topology.row_token.cpu().numpy()[rows[:n]], want.token) and np.all(rows[n:] == -1)
+
+
+@pytest.mark.parametrize("levels", [0, 3])
+@pytest.mark.parametrize(("t", "e", "k"), [
+    # alone, a lane reads its own row for up to 8 experts and from 512 groups of tokens on: 16 bytes at a time where
+    # rows are whole 16 bytes, else only few experts
+    (1, 8, 8), (65, 8, 2), (65, 9, 2), (32768, 20, 4), (32769, 20, 4), (32769, 64, 1), (32769, 45, 8), (32769, 49, 4),
+    (32769, 127, 16), (32833, 132, 16), (32833, 129, 5),
+])
+@pytest.mark.parametrize("offset", [0, 1])  # of the scores, in floats
+def test_topk_alone(t: int, e: int, k: int, levels: int, offset: int) -> None:
+    from sparsebench_amd import _C
+
+    scores = scores_of(t, e, levels)
+    dev = torch.empty(t * e + offset, device="cuda")[offset:].view(t, e).copy_(scores)
+    idx, weight = _C.router_topk_cuda(dev, k)
+    s = scores.numpy()
+    want = np.argsort(-s, axis=1, kind="stable")[:, :k]  # ties to the lower expert
+    picked = np.take_along_axis(s, want, axis=1)
+    total = np.zeros(t, dtype=np.float32)
+    for j in range(k):  # in pick order
+        total += picked[:, j]
+    assert np.array_equal(idx.cpu().numpy(), want)
+    assert np.array_equal(weight.cpu().numpy(), picked / total[:, None])
