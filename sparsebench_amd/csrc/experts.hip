@@ -33,7 +33,7 @@
 //
 // Every workgroup computes the same choice from tokens_per_expert
 // (expert_tiles_chosen): expert tiles for balanced routing, else row-block
-// tiles with sb_sdd's / sb_dsd's default tile shape. Both live in one kernel
+// tiles as wide as sb_sdd's and sb_dsd's widest. Both live in one kernel
 // so the choice costs nothing: two launches, one of them returning at once,
 // cost about 10 us each (every workgroup holds up to 160 KB of LDS while it
 // reads the counts). The row-block tiles run on the expert tiles' own code
@@ -426,7 +426,7 @@ __global__ void __launch_bounds__(CfgP::kThreads)
 
 // Expert tiles of the DSD: 4 waves, 256 columns, chunks of up to 256 rows.
 // Row-block tiles: 4 waves, 128 x CfgB::BN, every row of the row block read
-// and written, as sb_dsd's default tile does, except for an expert of one
+// and written, as sb_dsd's tiles do, except for an expert of one
 // row block, whose tile stops at its last real 32-row group (with few
 // tokens most row blocks are such experts, and mostly padding: 93% of the
 // rows at T = 512 of config 5); they run on the same tile code as the
@@ -623,7 +623,7 @@ int dispatch_sdd_layer(const void* x, const void* w1, const int32_t* row_token, 
                        void* out, int64_t num_tokens, int64_t d_model, int64_t ffn_dim, int64_t num_experts,
                        int64_t max_row_blocks, int64_t min_rows, int32_t apply_gelu, int32_t force,
                        hipStream_t stream) {
-  // The row-block tile is sb_sdd's for the shape (sdd_tile_for).
+  // The row-block tile is sb_sdd's widest for the shape (sdd_tile_for).
   if (sdd_tile_for(d_model, ffn_dim) == SddTile::kDeep)
     return launch_sdd_layer<SddDeepTile>(x, w1, row_token, row_block_expert, row_offsets, tokens_per_expert,
                                          padded_offsets, out, num_tokens, d_model, ffn_dim, num_experts,
@@ -754,7 +754,7 @@ int dsd_experts(const void* h, const void* w2, const int32_t* tokens_per_expert,
   if (max_row_blocks * kBS * d_model > (int64_t{1} << 62) || max_row_blocks * (d_model / kDsdBN) > kI32Max - 65536)
     return fail(SB_ERR_INVALID, "problem too large");
   const int32_t force = expert_gate_override();
-  // Row blocks forced: exactly sb_dsd version 5 (its default tile).
+  // Row blocks forced: exactly sb_dsd version 5.
   if (force == 2)
     return sb_dsd(h, w2, row_offsets, col_indices, out, max_row_blocks * (ffn_dim / kBS), num_experts * ffn_dim,
                   max_row_blocks, kBS, d_model, 0, stream);

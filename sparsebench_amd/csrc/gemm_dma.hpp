@@ -149,7 +149,7 @@ struct DmaCfg {
   static_assert(WTM % 32 == 0 && WTN % 32 == 0, "waves own whole 32 x 32 blocks");
   static_assert(kAInstr >= 1 && kABytes >= BM * kARowBytes, "the A area holds BM rows");
   static_assert(kBInstr >= 1 && kBInstr * kWaves * 1024 == kBBytes, "B step splits into whole 1 KB DMA rows");
-  static_assert(STAGES >= 2 && STAGES <= 16, "STAGES");
+  static_assert(STAGES >= 2 && STAGES <= 8, "STAGES");
   static_assert(kLdsAlloc <= 160 * 1024, "LDS");
   static_assert((APAIR ? kLaterLoadsOdd : kLaterLoads) <= 63, "vmcnt");
   static_assert(!APAIR || (BK == 32 && (STAGES == 3 || STAGES == 4) && (PIPE == 3 || PIPE == 4 || PIPE == 5)),

@@ -1,7 +1,7 @@
 // The layer kernels' tile schedules, compiled for the CPU: extern "C" shims
 // over the same __host__ __device__ functions the kernels call
 // (common.hpp: xcd_remap, split_tail, split_tail_slack, tile_coords;
-// dsd_tile.hpp: dsd_form;
+// dsd_tile.hpp: dsd_form; sdd_tile.hpp: sdd_form;
 // expert_chunks.hpp: balanced_chunk_tile, lpt_group_tile, pair_units_per_xcd,
 // pair_tile_for, narrow_width, may_be_narrow, narrow_tile_for), so
 // tests/test_tile_schedules.py and tests/test_narrow_tiles.py check the
@@ -10,6 +10,7 @@
 
 #include "dsd_tile.hpp"
 #include "expert_chunks.hpp"
+#include "sdd_tile.hpp"
 
 using namespace sb;
 
@@ -18,6 +19,10 @@ extern "C" int sbt_dsd_form(int64_t block_size, int64_t nnz, int64_t w_rows, int
                             int routed, int cus) {
   const DsdForm f = dsd_form(block_size, nnz, w_rows, num_row_blocks, d_model, routed != 0, cus);
   return f.width + (f.paired ? 1 : 0) + (f.deep ? 2 : 0);
+}
+
+extern "C" int sbt_sdd_form(int64_t num_row_blocks, int64_t d_model, int64_t ffn_dim, int cus) {
+  return static_cast<int>(sdd_form(num_row_blocks, d_model, ffn_dim, cus));
 }
 
 extern "C" int sbt_xcd_remap(int bid, int live) { return xcd_remap(bid, live); }

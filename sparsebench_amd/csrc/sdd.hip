@@ -92,11 +92,9 @@ extern "C" int sb_sdd(const void* x, const void* w1, const int32_t* row_token, c
       num_tokens * d_model > (int64_t{1} << 62) || num_row_blocks * 128 > kI32Max)
     return fail(SB_ERR_INVALID, "problem too large");
   const hipStream_t s = as_stream(stream);
-  // Fewer tiles than CUs: the narrower forms (fit_width).
   int cus = 0;
   if (const int rc = device_cus(&cus)) return rc;
-  const int width = fit_width(num_row_blocks, ffn_dim, cus);
-  const SddTile tile = width == 512 ? sdd_tile_for(d_model, ffn_dim) : width == 256 ? SddTile::kNarrow : SddTile::kHalf;
+  const SddTile tile = sdd_form(num_row_blocks, d_model, ffn_dim, cus);
   if (sdd_wide_x(num_tokens, d_model))
     return dispatch_sdd<true>(tile, x, w1, row_token, row_block_expert, row_offsets, out, num_tokens, d_model, ffn_dim,
                               num_experts, num_row_blocks, apply_gelu, s);

@@ -1,6 +1,6 @@
 // One SDD tile of a row block on the LDS-DMA main loop (gemm_dma.hpp): the
-// tile of the per-row-block kernel (sdd.hip), and that kernel's default
-// tile shape, which the MoE layer's SDD kernel (experts.hip) also uses.
+// tile of the per-row-block kernel (sdd.hip), and that kernel's tile shapes,
+// the widest of which the MoE layer's SDD kernel (experts.hip) also uses.
 #pragma once
 
 #include "expert_chunks.hpp"
@@ -152,6 +152,16 @@ enum class SddTile { kWide, kDeep, kNarrow, kHalf };
 inline SddTile sdd_tile_for(int64_t d_model, int64_t ffn_dim) {
   if (ffn_dim % 512 != 0) return SddTile::kNarrow;
   return d_model >= 4096 ? SddTile::kDeep : SddTile::kWide;
+}
+
+// sb_sdd's form: of the widest tiles the one for the shape, of fewer columns
+// when the grid has fewer tiles than CUs (fit_width).
+inline SddTile sdd_form(int64_t num_row_blocks, int64_t d_model, int64_t ffn_dim, int cus) {
+  switch (fit_width(num_row_blocks, ffn_dim, cus)) {
+    case 512: return sdd_tile_for(d_model, ffn_dim);
+    case 256: return SddTile::kNarrow;
+    default: return SddTile::kHalf;
+  }
 }
 
 // x of 2 GiB or more needs the 64-bit gather (SddDmaSrc's global form).

@@ -3,6 +3,7 @@ selects (128, 256, 512 columns), and the DSD's pairs of 64-row blocks: pairs
 with the same columns, neighbours with other columns or another block count,
 an odd last row block and dead ones, against the oracle."""
 
+import ctypes
 import math
 
 import numpy as np
@@ -11,6 +12,7 @@ import torch
 
 from oracle.moe_ref import dsd_rows, sdd_blocks
 from oracle.topology_ref import build_layout
+from sparsebench_amd import _lib
 
 pytestmark = pytest.mark.gpu
 
@@ -22,15 +24,30 @@ def routed(counts: list[int], seed: int) -> np.ndarray:
     return np.random.default_rng(seed).permutation(idx).reshape(-1, 1)
 
 
-@pytest.mark.parametrize(("counts", "d", "f"), [
-    # rows per expert; the row blocks and D choose the width
-    ([640, 300, 700], 8192, 256),       # 256 wide in pairs: 27 row blocks x 16 of 512 columns leave them idle at 512
-    ([4000, 1, 3900], 1536, 128),       # more tiles than CUs: pairs, 512 wide
-    ([2500, 2600, 2700], 768, 8192),    # the same, D % 512 != 0: 256 wide
-    ([4100, 63], 1536, 8192),           # pairs, 512 wide over a deep reduction
-    ([700, 650], 512, 256), ([70, 1, 64], 512, 256), ([9000], 1024, 64),
+@pytest.fixture(scope="module")
+def form():
+    """The launch's own rule, for 256 CUs: width + 1 in pairs + 2 deep."""
+    _lib.lib()  # torch's HIP runtime first
+    fn = ctypes.CDLL(str(_lib.LIB_PATH.with_name("libsparsebench_probe.so"))).sbt_dsd_form
+    fn.argtypes = [ctypes.c_int64] * 5 + [ctypes.c_int] * 2
+    return fn
+
+
+PAIRED, DEEP = 1, 2
+
+
+@pytest.mark.parametrize(("counts", "d", "f", "want"), [
+    # rows per expert; the row blocks and D choose the form
+    ([520], 8192, 256, 256 + PAIRED),               # 512 wide they leave CUs idle, in pairs 256 wide fit
+    ([2000, 2100], 1024, 256, 256 + PAIRED),        # the same, an odd row block of one expert
+    ([4000, 1, 3900], 1536, 128, 512),              # one round of pairs would be nearly full
+    ([4200, 250, 4300], 1024, 256, 512 + PAIRED),   # pairs leave room
+    ([8700, 130, 9000], 1024, 256, 512 + PAIRED),   # pairs are more than one round
+    ([2000, 2100, 2000], 768, 1024, 256 + PAIRED),  # D % 512 != 0
+    ([1050], 8192, 9216, 512 + PAIRED + DEEP),
+    ([700, 650], 512, 256, 128), ([70, 1, 64], 512, 256, 128), ([2600], 1536, 64, 256),
 ])
-def test_block_64_against_oracle(counts: list[int], d: int, f: int) -> None:
+def test_block_64_against_oracle(form, counts: list[int], d: int, f: int, want: int) -> None:
     from sparsebench_amd import _C
 
     e = len(counts)
@@ -38,8 +55,9 @@ def test_block_64_against_oracle(counts: list[int], d: int, f: int) -> None:
     g = torch.Generator().manual_seed(f)
     blocks = (torch.randn(lay.col_indices.size, 64, 64, generator=g) / math.sqrt(f)).bfloat16()
     w = torch.randn(e * f, d, generator=g).bfloat16()
-    dead = 3
+    dead = 1
     offsets = torch.cat([torch.as_tensor(lay.row_offsets), torch.full((dead,), int(lay.row_offsets[-1]))]).int()
+    assert form(64, blocks.shape[0], w.shape[0], offsets.numel() - 1, d, 1, 256) == want
     out = _C.dsd_cuda(blocks.cuda(), w.cuda(), offsets.cuda(), torch.as_tensor(lay.col_indices).cuda(), 1, routed=True)
     torch.testing.assert_close(out[: lay.num_rows].float().cpu(), dsd_rows(blocks.float(), w.float(), lay), **TOL)
     assert torch.all(out[lay.num_rows:] == 0)
@@ -119,8 +137,11 @@ def test_sdd_widths(counts: list[int], d: int, f: int) -> None:
     torch.testing.assert_close(out[: lay.col_indices.size].float().cpu(), sdd_blocks(x.float(), w1.float(), lay), **TOL)
 
 
-@pytest.mark.parametrize(("counts", "d", "f"), [([100, 300], 256, 256), ([100, 300], 8192, 256), ([300, 200], 32768, 128)])
-def test_dsd_widths_block_128(counts: list[int], d: int, f: int) -> None:
+@pytest.mark.parametrize(("counts", "d", "f", "want"), [
+    ([100, 300], 256, 256, 128), ([100, 300], 8192, 256, 128), ([400, 300], 8192, 256, 256),
+    ([300, 200], 32768, 128, 512),
+])
+def test_dsd_widths_block_128(form, counts: list[int], d: int, f: int, want: int) -> None:
     from sparsebench_amd import _C
 
     e = len(counts)
@@ -128,6 +149,7 @@ def test_dsd_widths_block_128(counts: list[int], d: int, f: int) -> None:
     g = torch.Generator().manual_seed(f + d)
     blocks = (torch.randn(lay.col_indices.size, 128, 128, generator=g) / math.sqrt(f)).bfloat16()
     w = torch.randn(e * f, d, generator=g).bfloat16()
+    assert form(128, blocks.shape[0], w.shape[0], len(lay.row_offsets) - 1, d, 0, 256) == want
     out = _C.dsd_cuda(blocks.cuda(), w.cuda(), torch.as_tensor(lay.row_offsets).int().cuda(),
                       torch.as_tensor(lay.col_indices).cuda(), 1)
     torch.testing.assert_close(out.float().cpu(), dsd_rows(blocks.float(), w.float(), lay), **TOL)

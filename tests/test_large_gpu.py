@@ -106,6 +106,28 @@ def test_sdd_accepts_x_over_2gib(entry: str, form: str) -> None:
         torch.testing.assert_close(got, want, rtol=1.6e-2, atol=1.6e-2, msg=f"row {r} token {tok}")
 
 
+def test_sdd_of_few_copies_of_x_over_2gib() -> None:
+    # So few row blocks that sb_sdd takes its 128-wide tiles, gathering x with 64-bit addresses.
+    from sparsebench_amd.routing import route_assigned
+    from sparsebench_amd.spmm import sdd
+
+    x, _, _, w1, _ = wide_inputs()
+    e, f, t = WIDE.num_experts, WIDE.ffn_dim, WIDE.num_tokens
+    token = torch.cat([torch.arange(t - 150, t), torch.arange(50)]).int().cuda()
+    expert = (torch.arange(200) % 3).int().cuda()
+    topo = route_assigned(token, expert, t, e, f, 128).topology
+    assert topo.row_block_expert.numel() * (f // 128) <= 256
+    h = sdd(x, w1, topo)
+    rows = topo.copy_row.long()
+    fb = f // 128
+    got = h.view(-1, fb, 128, 128)[rows // 128, :, rows % 128, :].reshape(200, f).float().cpu()
+    # One product an expert, in fp32 on the CPU (its error is far below bf16's).
+    for i in range(3):
+        own = torch.arange(i, 200, 3)
+        want = gelu_erf((x[token[own.cuda()].long()].float().cpu() @ w1[i].float().cpu()).double()).float()
+        torch.testing.assert_close(got[own], want, rtol=1.6e-2, atol=1.6e-2)
+
+
 def test_layer_with_x_over_2gib() -> None:
     from sparsebench_amd.moe import moe_forward
 
