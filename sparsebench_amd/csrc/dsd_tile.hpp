@@ -147,16 +147,19 @@ __device__ __forceinline__ void dsd_pair_tile(uint8_t* __restrict__ lds, int bid
                                               int32_t num_slices, int32_t zero_dead_rows, int32_t group) {
   using ML = DmaMainloop<Cfg>;
   constexpr int BN = Cfg::BN;
-  // The first workgroups of all pairs' slices, then the second ones.
+  // The second workgroups of all pairs' slices, then the first ones: most of the
+  // second ones end at once, and none of them then waits for a CU behind the
+  // first ones' tiles (D = 1024, F = 1024, E = 8, 50 row blocks: 0.89 of the time
+  // of row blocks one by one, and 1.0 with the second ones last).
   const int pairs = (num_row_blocks + 1) / 2;
-  const int which = uniform(bid / (pairs * num_slices));
+  const int which = bid < pairs * num_slices ? 1 : 0;
   const int live_rb = zero_dead_rows ? num_row_blocks : live_row_blocks(row_offsets, num_row_blocks);
   const int live = (live_rb + 1) / 2;
   // A pair's second ones, its slices, one by one over the XCDs: only those of
   // row blocks alone have work, and with all of them on one XCD that needs a
   // round of its own (D = 4096, F = 1024, E = 2, 18 row blocks: 0.83 of the time
   // of row blocks one by one, 1.37 in the order of the first ones).
-  const int id = bid - which * pairs * num_slices;
+  const int id = which == 0 ? bid - pairs * num_slices : bid;
   int pair, slice;
   if (which == 0) {
     tile_coords(xcd_remap(id, live * num_slices), live, num_slices, group, &pair, &slice);
@@ -164,7 +167,7 @@ __device__ __forceinline__ void dsd_pair_tile(uint8_t* __restrict__ lds, int bid
     pair = uniform(id / num_slices);
     slice = id - pair * num_slices;
   }
-  if (pair >= pairs || which > 1) return;
+  if (pair >= pairs) return;
   const int n0 = slice * BN;
   int rb = 2 * pair;
 
@@ -249,16 +252,16 @@ struct DsdForm {
 // expert's end. Pairs are taken when they let 512-wide tiles that leave CUs
 // idle become 256-wide ones (at least 4 row blocks an expert), or when there
 // are more tiles than CUs and at least 8 row blocks an expert; the row block
-// count may be a worst case, up to E more than there are. But the tiles of row
-// blocks alone come last, and where the pairs leave few CUs free one of them
-// may wait for a round of its own: so the pairs must leave three CUs of eight
-// and the others fill at most two, or the pairs be more than one round
-// themselves. Pairs against one by one, F = 1024 and 4096, E = 2 to 16, P tiles
-// of pairs on 256 CUs: up to P = 160 0.59-0.90 of the time (1.26 once in 211
-// routings); P = 168-256 0.62-0.97 or, by the routing's chance, 1.06-1.46;
-// more 0.64-0.95. D = 1024, 79 row blocks, E = 20 1.41. D = 4096, 79 row blocks 138 against 153 us; D = 512 (256 and 128
-// wide) 29 against 44; 3 row blocks an expert (D = 1024, F = 4096, E = 64) 174
-// against 188.
+// count may be a worst case, up to E more than there are. But where the pairs
+// leave few CUs free, the tiles of row blocks alone may cost a round of their
+// own: so the pairs must leave some of the CUs, by the number of experts, or be
+// more than one round themselves. Pairs against one by one, F = 1024 and 4096,
+// P tiles of pairs on 256 CUs: up to P = 160 0.59-0.92 of the time (1.26 once in
+// 211 routings); P = 168-256 0.60-0.92 or, by the routing's chance, 1.06-1.42
+// (E = 2 from P = 232 on, E = 4 from 200, E = 8 and 16 from 170); more
+// 0.64-0.95. D = 1024, 79 row blocks, E = 20 1.41. D = 4096, 79 row blocks 138
+// against 153 us; D = 512 (256 and 128 wide) 29 against 44; 3 row blocks an
+// expert (D = 1024, F = 4096, E = 64) 174 against 188.
 // Of any other BSR the neighbours' columns differ, and every row block would
 // cost a whole tile for its half: none in pairs (64 column blocks, half of
 // them in each row: 256 row blocks, D = 1024 129 one by one against 147 us in
@@ -276,7 +279,9 @@ inline DsdForm dsd_form(int64_t block_size, int64_t nnz, int64_t w_rows, int64_t
   const int paired = fit_width((num_row_blocks + experts) / 2, d_model, cus);
   const int64_t least = num_row_blocks - experts;  // row blocks, of a routing layout's worst case
   const int64_t slices = d_model / paired;
-  const bool one_round = (num_row_blocks + 1) / 2 * slices <= cus * 5 / 8 && (experts - 1) * slices <= cus / 4;
+  const int eighths = experts <= 2 ? 7 : experts <= 4 ? 6 : 5;
+  const bool one_round =
+      (num_row_blocks + 1) / 2 * slices <= cus * eighths / 8 && (experts - 1) * slices <= cus / 4;
   const bool rounds = least / 2 * slices > cus;
   const bool narrower = single == 512 && paired == 256 && num_row_blocks >= 4 * experts && one_round;
   const bool many = least * (d_model / single) > cus && num_row_blocks >= 8 * experts && (one_round || rounds);

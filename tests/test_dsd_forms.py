@@ -39,7 +39,8 @@ def test_pairs_only_for_routing_layouts(form, rb: int, cols: int, d: int, share:
 
 @pytest.mark.parametrize(("e", "d", "rows", "paired"), [
     # rows: row blocks that hold rows; one expert's odd one out and the worst case add up to E more
-    (16, 1024, 63, True), (2, 768, 104, True), (1, 512, 158, True),     # the pairs leave three CUs of eight
+    (16, 1024, 63, True), (2, 768, 104, True), (1, 512, 158, True),     # the pairs leave CUs enough
+    (2, 768, 146, True), (4, 768, 122, True), (8, 768, 120, False),     # the fewer, the more experts
     (4, 1536, 66, False), (2, 768, 158, False), (16, 512, 400, False),  # one round, nearly full
     (16, 1024, 122, False),                                             # one by one may be one round
     (20, 1024, 80, False),                                              # many row blocks alone
