@@ -605,7 +605,8 @@ __global__ void __launch_bounds__(kSelectThreads)
 // workgroups past the words write the block-sparse layout. (Separate kernels
 // for counts, their scan, the list and the layout took 4.7 + 5.4 + 4.7 + 4.6
 // us at T = 4096, E = 64, each little more than its launch; this takes
-// 6.1.)
+// 6.1. The whole rounding at T = 4096, before and now: E = 300, k = 4 137 and 84
+// us; E = 512, k = 8 232 and 167; E = 1000, k = 8 338 and 301.)
 template <int PER>
 __global__ void __launch_bounds__(kEmitThreads)
     router_emit_kernel(const float* __restrict__ scores, int64_t num_tokens, int32_t num_experts,
