@@ -767,14 +767,16 @@ int launch_topk(const float* scores, int64_t num_tokens, int32_t num_experts, in
   const int kmax = k <= 1 ? 1 : k <= 2 ? 2 : k <= 4 ? 4 : k <= 8 ? 8 : 16;
   const int forced = test_hook(SB_HOOK_TOPK_KERNEL);
   if (forced == 2 || (forced != 1 && kmax * num_experts <= 8192)) {
-    // Alone, the direct form for up to 8 experts (T = 4096, k = 2: E = 8 2.8
-    // against 3.8 us, E = 16 in tiles 4.0 and direct 4.2) and from 512 groups on
-    // (T = 131072, k = 2: E = 32 5.5 against 13.1; T = 32768, E = 64 7.0 in tiles,
-    // 10.8 direct), where a lane reads 16 bytes at a time or few at all
-    // (T = 300000, E = 129, k = 4 in tiles 124, direct 650).
+    // Alone, the direct form where a row takes few loads of 16 bytes and little
+    // work (T = 4096, direct against tiles: E = 8, k = 2 2.8 and 3.8 us; E = 16,
+    // k = 2 3.0 and 4.0; E = 60, k = 4 8.4 and 10.2; but E = 128, k = 8 31.8 and
+    // 30.1; rows read 4 bytes at a time E = 33, k = 2 6.0 and 4.9) and from 512
+    // groups on (T = 131072, E = 32, k = 2 5.5 and 13.1), there of rows that are
+    // not whole 16 bytes only short ones (T = 300000, E = 129, k = 4 650 and 124).
     const bool wide = num_experts % 4 == 0 && aligned16(scores);
     const bool direct = shifted == nullptr && chunk_counts == nullptr &&
-                        (num_experts <= 8 || (groups > 512 && (wide || num_experts <= std::max(48, 8 * kmax))));
+                        (num_experts <= 8 || (wide && kmax * num_experts <= 256) ||
+                         (groups > 512 && (wide || num_experts <= std::max(48, 8 * kmax))));
     // Rows read 4 bytes at a time are read again and again from L1, which holds
     // those of a few waves: LDS that the kernel does not use keeps a CU at 13
     // (T = 300000, E = 45, k = 8 165 us without, 88 with).

@@ -45,9 +45,9 @@ def test_list_matches_oracle(t: int, e: int, k: int, tile: int, levels: int) -> 
 
 @pytest.mark.parametrize("levels", [0, 3])
 @pytest.mark.parametrize(("t", "e", "k"), [
-    # alone, a lane reads its own row for up to 8 experts and from 512 groups of tokens on: 16 bytes at a time where
-    # rows are whole 16 bytes, else only few experts
-    (1, 8, 8), (65, 8, 2), (65, 9, 2), (32768, 20, 4), (32769, 20, 4), (32769, 64, 1), (32769, 45, 8), (32769, 49, 4),
+    # alone, a lane reads its own row for up to 8 experts, for short rows of whole 16 bytes, and from 512 groups of
+    # tokens on, there of other rows only short ones
+    (1, 8, 8), (65, 8, 2), (65, 9, 2), (65, 64, 4), (65, 64, 5), (300, 20, 3), (64, 132, 1), (32768, 20, 4), (32769, 20, 4), (32769, 64, 1), (32769, 45, 8), (32769, 49, 4),
     (32769, 127, 16), (32833, 132, 16), (32833, 129, 5),
 ])
 @pytest.mark.parametrize("offset", [0, 1])  # of the scores, in floats
